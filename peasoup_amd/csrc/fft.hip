@@ -361,16 +361,7 @@ __global__ void __launch_bounds__(256) k_untangle(float2* __restrict__ X, uint64
   }
 }
 
-// C2R pre-pass, out of place: W[k] = conj( (Xk + Xm*) + i conj(W_n^k) (Xk - Xm*) )
-// for k in [0, M), with Xm = X[M-k].  The conjugate feeds the forward passes.
-__device__ inline float2 tangle_one(float2 xk, float2 xm, float2 w) {
-  const float2 s = make_float2(xk.x + xm.x, xk.y - xm.y);
-  const float2 d = make_float2(xk.x - xm.x, xk.y + xm.y);
-  const float2 cd = cmul(make_float2(w.x, -w.y), d);
-  const float2 z = make_float2(s.x - cd.y, s.y + cd.x);
-  return make_float2(z.x, -z.y);
-}
-
+// C2R pre-pass, out of place: W[k] = tangle_one(X[k], X[M-k], W_n^k), k in [0, M).
 __global__ void __launch_bounds__(256) k_tangle(const float2* __restrict__ X, float2* __restrict__ W, uint64_t M,
                                                 int64_t in_tr, int64_t out_tr, RootTable rt) {
   const float2* x = X + (int64_t)blockIdx.y * in_tr;
@@ -810,7 +801,8 @@ int build_passes(psx_fft_plan* p, bool device_tables) {
 namespace psx {
 namespace fft {
 
-int plan_create_with(uint64_t n, int kind, uint32_t batch, const Decomp* forced, psx_fft_plan** out) {
+int plan_create_with(uint64_t n, int kind, uint32_t batch, const Decomp* forced, psx_fft_plan** out,
+                     bool own_work) {
   PSX_REQUIRE(out, "psx_fft_plan_create: null plan");
   *out = nullptr;
   PSX_REQUIRE(kind == PSX_FFT_R2C || kind == PSX_FFT_C2R, "psx_fft_plan_create: bad kind %d", kind);
@@ -840,7 +832,7 @@ int plan_create_with(uint64_t n, int kind, uint32_t batch, const Decomp* forced,
   }
   rc = build_passes(p, true);
   if (!rc) {
-    const bool need_work = (kind == PSX_FFT_C2R) || p->d.npass > 1;
+    const bool need_work = own_work && ((kind == PSX_FFT_C2R) || p->d.npass > 1);
     if (need_work) {
       hipError_t e = hipMalloc(&p->work, sizeof(float2) * p->M * batch);
       if (e != hipSuccess) rc = psx::fail(PSX_ERR_ALLOC, "FFT work buffer: %s", hipGetErrorString(e));
@@ -882,6 +874,23 @@ int plan_exec(psx_fft_plan* p, const void* in, void* out, hipStream_t hs) {
     const unsigned g = psx::grid_for(p->M / 2 + 1, tb);
     k_untangle<<<dim3(g, p->batch), tb, 0, hs>>>((float2*)out, p->M, (int64_t)p->nb, p->rt);
     PSX_CHECK_LAUNCH("k_untangle");
+  }
+  return PSX_OK;
+}
+
+int exec_passes(psx_fft_plan* p, const void* in, float2* work, void* out, uint32_t ntr, hipStream_t hs) {
+  if (ntr < 1 || ntr > p->batch || !out || !work || (p->kind == PSX_FFT_R2C && !in))
+    return psx::fail(PSX_ERR_ARG, "exec_passes: bad arguments");
+  const uint64_t cap = p->M * ntr;
+  for (PassLaunch& L : p->passes) {
+    PassArgs a = L.a;
+    a.in = L.src == 0 ? (const float2*)in : work;
+    a.out = L.dst == 2 ? (float2*)out : work;
+    if (L.dst == 2) a.out_tr = (int64_t)p->M;
+    int rc = check_pass_bounds(L, a, ntr, cap, cap, 0);
+    if (rc) return rc;
+    hipLaunchKernelGGL(L.k->fn, dim3(L.gx, L.gy, ntr), dim3(L.k->threads), L.k->lds, hs, a);
+    PSX_CHECK_LAUNCH("k_fft_pass");
   }
   return PSX_OK;
 }

@@ -45,6 +45,16 @@ __device__ inline float2 untangle_one(float2 zk, float2 zm, float2 w) {
   return make_float2(e.x + 0.5f * wd.y, e.y - 0.5f * wd.x);
 }
 
+// C2R input of one bin: conj((xk + conj(xm)) + i conj(w) (xk - conj(xm))),
+// xm = X[M-k]; the conjugate feeds the forward passes.
+__device__ inline float2 tangle_one(float2 xk, float2 xm, float2 w) {
+  const float2 s = make_float2(xk.x + xm.x, xk.y - xm.y);
+  const float2 d = make_float2(xk.x - xm.x, xk.y + xm.y);
+  const float2 cd = cmul(make_float2(w.x, -w.y), d);
+  const float2 z = make_float2(s.x - cd.y, s.y + cd.x);
+  return make_float2(z.x, -z.y);
+}
+
 // Bin k in [0, M] of the untangled spectrum, computed exactly as the in-place
 // untangle pass does (so fused consumers see identical values).
 __device__ inline float2 untangled_bin(const float2* __restrict__ z, uint64_t M, uint64_t k, const RootTable& rt) {
@@ -55,8 +65,15 @@ __device__ inline float2 untangled_bin(const float2* __restrict__ z, uint64_t M,
   return untangle_one(z[k], z[M - k], make_float2(-w.x, w.y));
 }
 
-int plan_create_with(uint64_t n, int kind, uint32_t batch, const Decomp* forced, psx_fft_plan** out);
+// own_work = false: no work buffer (for exec_passes, which is given one).
+int plan_create_with(uint64_t n, int kind, uint32_t batch, const Decomp* forced, psx_fft_plan** out,
+                     bool own_work = true);
 int plan_exec(psx_fft_plan* p, const void* in, void* out, hipStream_t s);
+// The complex passes alone for the first ntr transforms of a plan, without
+// the (un)tangle pass: R2C in (ntr x n real samples) -> out (half-length
+// spectra, stride M); C2R work (tangled spectra, stride M) -> out (ntr x n
+// samples).  work: ntr x M complex, the passes' intermediate.
+int exec_passes(psx_fft_plan* p, const void* in, float2* work, void* out, uint32_t ntr, hipStream_t s);
 // Forward complex passes of an R2C plan whose first pass reads trial
 // blockIdx.z through the resampler (descs); writes the half-length complex
 // spectra Z (trial stride M) to zout without untangling.

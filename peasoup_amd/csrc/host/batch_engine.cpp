@@ -33,6 +33,13 @@ void halloc(T** p, uint64_t n) {
   hip_ok(hipHostMalloc((void**)p, sizeof(T) * (n ? n : 1), hipHostMallocDefault), "hipHostMalloc");
 }
 int64_t round_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
+// Device bytes counted for the prologue: two half-length spectra and about as
+// much again of medians and work, plans and tables.
+uint64_t prologue_bytes(uint64_t M) {
+  const uint64_t nb = M + 1;
+  return nb * (sizeof(float2) + 2 * sizeof(float)) + nb / 4 * sizeof(float) + 2 * M * sizeof(float2) +
+         16 * 1024 * 1024;
+}
 }  // namespace
 
 uint64_t Engine::device_bytes(uint64_t N, uint32_t B, uint32_t cap) {
@@ -43,9 +50,20 @@ uint64_t Engine::device_bytes(uint64_t N, uint32_t B, uint32_t cap) {
   b += (pst * B + kHarmWaveBins) * sizeof(float);  // P
   b += (uint64_t)bound_stride((int64_t)pst) * B * sizeof(uint16_t);  // Q
   b += 2 * (uint64_t)cap * sizeof(Cand16);
-  b += nb * (sizeof(float2) + 2 * sizeof(float)) + nb / 4 * sizeof(float);  // prologue X, A, median
-  b += 2 * M * sizeof(float2) + 16 * 1024 * 1024;                          // prologue plans + tables
+  b += prologue_bytes(M);
   return b;
+}
+
+// DM trials per prologue group: 2^25 samples (one launch of each pass then
+// takes long against its launch, and a group's spectra are at most 512 MB),
+// at most 64, and no more device memory than device_bytes counts: the
+// prologue's share and, in the fused form, the spectra P it never allocates.
+static uint32_t prologue_group_of(uint64_t N, uint32_t B, int64_t pstride, bool fused) {
+  const uint64_t M = N / 2;
+  const uint64_t room = prologue_bytes(M) - 4 * 1024 * 1024 + (fused ? (uint64_t)pstride * B * sizeof(float) : 0);
+  uint32_t G = (uint32_t)std::min<uint64_t>(64, std::max<uint64_t>(1, (1ull << 25) / N));
+  while (G > 1 && 2 * M * G * sizeof(float2) + psx::prologue::work_bytes(N, G) > room) --G;
+  return G;
 }
 
 Engine::Engine(const psx_search_args& a, const EngineOptions& opt, hipStream_t stream)
@@ -110,16 +128,14 @@ Engine::Engine(const psx_search_args& a, const EngineOptions& opt, hipStream_t s
   }
   if (win.hi <= win.lo) win.lo = win.hi = 0;
   win.thr = args.min_snr;
-  // prologue resources (plain path)
-  psx_ok(psx_fft_plan_create(N, PSX_FFT_R2C, 1, &p_r2c), "prologue R2C plan");
-  psx_ok(psx_fft_plan_create(N, PSX_FFT_C2R, 1, &p_c2r), "prologue C2R plan");
-  dalloc(&X, nb);
-  dalloc(&A, nb);
-  dalloc(&med, nb);
-  dalloc(&med_work, psx_deredden_work_floats(nb));
+  // prologue resources: the plain path's default plans
+  const uint32_t G = prologue_group_of(N, B, pstride, fused);
+  psx_ok(psx::fft::plan_create_with(N, PSX_FFT_R2C, G, nullptr, &p_r2c, false), "prologue R2C plan");
+  psx_ok(psx::fft::plan_create_with(N, PSX_FFT_C2R, G, nullptr, &p_c2r, false), "prologue C2R plan");
+  dalloc(&pz, M * G);
+  dalloc(&pw, M * G);
+  psx_ok(psx::prologue::work_create(N, G, pro), "prologue work");
   dalloc((uint8_t**)&red_work, psx_reduce_work_bytes());
-  dalloc(&d_base, 1);
-  dalloc(&d_sums, 1);
 }
 
 Engine::~Engine() {
@@ -142,36 +158,52 @@ Engine::~Engine() {
   psx_fft_plan_destroy(plan);
   psx_fft_plan_destroy(p_r2c);
   psx_fft_plan_destroy(p_c2r);
-  (void)hipFree(X);
-  (void)hipFree(A);
-  (void)hipFree(med);
-  (void)hipFree(med_work);
+  (void)hipFree(pz);
+  (void)hipFree(pw);
+  psx::prologue::work_destroy(pro);
   (void)hipFree(red_work);
-  (void)hipFree(d_base);
-  (void)hipFree(d_sums);
 }
 
-void Engine::prologue(const float* d_series, uint64_t n_real, float* d_tim, float* mean, float* std,
-                      const Zapper* zap) {
-  // pipeline_multi.cu:170-238
-  const uint64_t ncopy = std::min<uint64_t>(n_real, N);
-  if (d_series != d_tim) hip_ok(hipMemcpyAsync(d_tim, d_series, ncopy * sizeof(float), hipMemcpyDeviceToDevice, s),
-                                "prologue copy");
-  psx_ok(psx_remove_baseline(d_tim, ncopy, red_work, s), "remove_baseline");
-  if (N > n_real) psx_ok(psx_fill(d_tim, n_real, N, 0.0f, s), "fill");
+void Engine::set_zap(const Zapper* zap, hipStream_t ps) {
+  pro_zap = zap && zap->size() > 0;
+  if (!pro_zap) return;
   const float tobs = (unsigned int)N * args.tsamp;
   const float bin_width = 1.0 / tobs;
-  psx_ok(psx_fft_exec(p_r2c, d_tim, X, s), "prologue R2C");
-  psx_ok(psx_form_amplitude(X, A, nb, s), "form");
-  psx_ok(psx_deredden_median(A, nb, (double)bin_width, 0.05f, 0.5f, med, med_work, s), "calculate_median");
-  psx_ok(psx_divide_c_by_f(X, med, nb, s), "deredden");
-  if (zap) zap->zap_on(X, bin_width, nb, s);
-  psx_ok(psx_form_interbin(X, A, nb, s), "form_interpolated");
-  float m = 0, r = 0;
-  psx_ok(psx_mean_rms(A, nb, 0, &m, &r, red_work, s), "stats");
-  *mean = m;
-  *std = std::sqrt(r * r - m * m);
-  psx_ok(psx_fft_exec(p_c2r, X, d_tim, s), "prologue C2R");
+  psx_ok(psx::prologue::zap_mask(pro, zap->get_device_birdies(), zap->get_device_widths(), (uint32_t)zap->size(),
+                                 bin_width, ps),
+         "zap list");
+}
+
+void Engine::prologue_async(const float* series, uint64_t stride, uint64_t n_real, float* tims, uint32_t ndm,
+                            PrologueResult* res, hipStream_t ps) {
+  // pipeline_multi.cu:170-238
+  psx_ok(psx::prologue::baseline(pro, series, (int64_t)stride, std::min<uint64_t>(n_real, N), tims, ndm, ps),
+         "remove_baseline");
+  prologue_spectra(tims, ndm, res, ps);
+}
+
+// From the series without their baselines to the dereddened ones.
+void Engine::prologue_spectra(float* tims, uint32_t ndm, PrologueResult* res, hipStream_t ps) {
+  const float tobs = (unsigned int)N * args.tsamp;
+  const float bin_width = 1.0 / tobs;
+  psx_ok(psx::fft::exec_passes(p_r2c, tims, pw, pz, ndm, ps), "prologue R2C");
+  psx_ok(psx::prologue::spectra(pro, pz, pw, psx::fft::root_table(p_r2c), (double)bin_width, 0.05f, 0.5f, pro_zap,
+                                ndm, ps),
+         "prologue spectra");
+  hip_ok(hipMemcpyAsync(res, pro.res, ndm * sizeof(PrologueResult), hipMemcpyDeviceToHost, ps), "stats copy");
+  psx_ok(psx::fft::exec_passes(p_c2r, nullptr, pw, tims, ndm, ps), "prologue C2R");
+}
+
+void Engine::prologue(const float* d_series, uint64_t n_real, float* d_tim, float* mean, float* std, hipStream_t ps) {
+  const uint64_t ncopy = std::min<uint64_t>(n_real, N);
+  if (d_series != d_tim)
+    hip_ok(hipMemcpyAsync(d_tim, d_series, ncopy * sizeof(float), hipMemcpyDeviceToDevice, ps), "prologue copy");
+  psx_ok(psx_remove_baseline(d_tim, ncopy, red_work, ps), "remove_baseline");
+  if (N > n_real) psx_ok(psx_fill(d_tim, n_real, N, 0.0f, ps), "fill");
+  PrologueResult res;
+  prologue_spectra(d_tim, 1, &res, ps);
+  hip_ok(hipStreamSynchronize(ps), "prologue");
+  stats_of(res, mean, std);
 }
 
 // Spectrum pass: from the natural half-length spectra, or from the
@@ -295,28 +327,6 @@ void Engine::harmonics(Slot& sl, uint32_t n) {
   } else {
     psx_ok(launch_harm_peaks(P, pstride, win, F, sl.d_desc, n, sl.d_cands, cap, sl.d_count, s), "harm_peaks");
   }
-}
-
-void Engine::prologue_async(const float* d_series, uint64_t n_real, float* d_tim, PrologueResult* res,
-                            hipStream_t ps, const Zapper* zap) {
-  // prologue() step for step, on ps
-  const uint64_t ncopy = std::min<uint64_t>(n_real, N);
-  if (d_series != d_tim)
-    hip_ok(hipMemcpyAsync(d_tim, d_series, ncopy * sizeof(float), hipMemcpyDeviceToDevice, ps), "prologue copy");
-  psx_ok(psx::remove_baseline_async(d_tim, ncopy, red_work, d_base, kBaselineSteps, ps), "remove_baseline");
-  if (N > n_real) psx_ok(psx_fill(d_tim, n_real, N, 0.0f, ps), "fill");
-  const float tobs = (unsigned int)N * args.tsamp;
-  const float bin_width = 1.0 / tobs;
-  psx_ok(psx_fft_exec(p_r2c, d_tim, X, ps), "prologue R2C");
-  psx_ok(psx_form_amplitude(X, A, nb, ps), "form");
-  psx_ok(psx_deredden_median(A, nb, (double)bin_width, 0.05f, 0.5f, med, med_work, ps), "calculate_median");
-  psx_ok(psx_divide_c_by_f(X, med, nb, ps), "deredden");
-  if (zap) zap->zap_on(X, bin_width, nb, ps);
-  psx_ok(psx_form_interbin(X, A, nb, ps), "form_interpolated");
-  psx_ok(psx::sum_sq_async(A, 0, nb, red_work, d_sums, ps), "stats");
-  hip_ok(hipMemcpyAsync(&res->base, d_base, sizeof(BaselineState), hipMemcpyDeviceToHost, ps), "baseline state");
-  hip_ok(hipMemcpyAsync(&res->sums, d_sums, sizeof(double2), hipMemcpyDeviceToHost, ps), "stats copy");
-  psx_ok(psx_fft_exec(p_c2r, X, d_tim, ps), "prologue C2R");
 }
 
 // psx_mean_rms's arithmetic on the sums, then prologue()'s std.

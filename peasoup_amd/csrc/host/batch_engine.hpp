@@ -16,7 +16,7 @@
 
 #include "batch.hpp"
 #include "fft_plan.hpp"
-#include "reduce_async.hpp"
+#include "prologue.hpp"
 #include "peasoup/candidates.hpp"
 #include "peasoup/transforms.hpp"
 #include "psx.h"
@@ -33,12 +33,9 @@ struct TrialWork {
   int dm_idx;
 };
 
-// Results of an asynchronous prologue, written by the device into pinned
-// host memory: the baseline loop's state and the interbinned spectrum's sums.
-struct PrologueResult {
-  BaselineState base;
-  double2 sums;  // (sum x, sum x^2) over the nb bins
-};
+// Results of an asynchronous prologue, copied to pinned host memory: the
+// baseline loop's state and the interbinned spectrum's sums.
+using PrologueResult = psx::prologue::Result;
 
 // Trials per fused batch when the caller leaves it to the library: 64 up to
 // 2^26 samples (the tuned choice on MI355X from 2^20 to 2^26; 1.9% faster
@@ -108,22 +105,25 @@ class Engine {
   // True when collect() would return without waiting on the device.
   bool ready_or_done();
 
-  // Worker prologue (pipeline_multi.cu:170-238) for one DM with the plain
-  // kernels: d_series (n_real samples) -> d_tim (N samples), mean/std.
-  // zap (optional) removes birdies after dereddening (pipeline_multi.cu:222-226).
-  void prologue(const float* d_series, uint64_t n_real, float* d_tim, float* mean, float* std,
-                const Zapper* zap = nullptr);
-  // The same prologue enqueued on stream ps with no host round trip: the
-  // baseline loop runs kBaselineSteps device iterations and the statistics
-  // arrive in *res (pinned host memory) when ps reaches them.  Consecutive
-  // calls must share ps (they reuse the prologue buffers in order).  If
-  // res->base.done is 0 once ps has passed the call, the baseline loop had
-  // not stopped: redo the DM with prologue().  stats_of turns *res into the
-  // (mean, std) prologue() returns.
-  static constexpr int kBaselineSteps = 4;
-  void prologue_async(const float* d_series, uint64_t n_real, float* d_tim, PrologueResult* res, hipStream_t ps,
-                      const Zapper* zap = nullptr);
+  // Worker prologue (pipeline_multi.cu:170-238) of up to prologue_group() DMs,
+  // enqueued on stream ps with no host round trip: series (DM d at
+  // series + d*stride, n_real samples; may be tims itself with stride N) ->
+  // tims (N samples per DM).  The baseline loop runs kBaselineSteps device
+  // iterations and the statistics arrive in res[0..ndm) (pinned host memory)
+  // when ps reaches them.  Consecutive calls must share ps or be ordered (they
+  // reuse the prologue buffers).  If res[d].base.done is 0 once ps has passed
+  // the call, the baseline loop had not stopped: redo the DM with prologue().
+  // stats_of turns a result into the (mean, std) prologue() returns.
+  uint32_t prologue_group() const { return pro.G; }
+  void prologue_async(const float* series, uint64_t stride, uint64_t n_real, float* tims, uint32_t ndm,
+                      PrologueResult* res, hipStream_t ps);
   void stats_of(const PrologueResult& res, float* mean, float* std) const;
+  // The prologue of one DM with the host-driven baseline loop, complete when
+  // it returns.
+  void prologue(const float* d_series, uint64_t n_real, float* d_tim, float* mean, float* std, hipStream_t ps);
+  // The birdies that later prologues on ps remove after dereddening
+  // (pipeline_multi.cu:222-226); nullptr: none.
+  void set_zap(const Zapper* zap, hipStream_t ps);
 
   // Average duration of each launch of one batch of n trials, timed with HIP
   // events on the engine stream over `reps` repetitions (after one warm-up).
@@ -185,16 +185,16 @@ class Engine {
   int next_slot = 0;
   std::vector<std::vector<std::vector<Candidate>>> ready;  // collected early by submit()
 
-  // prologue resources
+  // prologue resources: plans without work buffers of their own, two buffers
+  // of a group's half-length spectra, and the kernels' work
+  void prologue_spectra(float* tims, uint32_t ndm, PrologueResult* res, hipStream_t ps);
   psx_fft_plan* p_r2c = nullptr;
   psx_fft_plan* p_c2r = nullptr;
-  psx_c32* X = nullptr;
-  float* A = nullptr;
-  float* med = nullptr;
-  float* med_work = nullptr;
+  float2* pz = nullptr;
+  float2* pw = nullptr;
+  psx::prologue::Work pro;
+  bool pro_zap = false;
   void* red_work = nullptr;
-  BaselineState* d_base = nullptr;
-  double2* d_sums = nullptr;
 };
 
 }  // namespace batch

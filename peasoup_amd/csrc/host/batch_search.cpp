@@ -223,7 +223,8 @@ extern "C" int psx_batch_profile(const psx_search_args* args, const psx_batch_op
     std::unique_ptr<Zapper> zap;
     if (args->nbirdies) zap.reset(new Zapper(args->birdie_freq, args->birdie_width, args->nbirdies, s));
     float mean, sd;
-    eng->prologue(d_series, nsamps, d_tim, &mean, &sd, zap.get());
+    eng->set_zap(zap.get(), s);
+    eng->prologue(d_series, nsamps, d_tim, &mean, &sd, s);
     const uint32_t n = std::min(naccs, eng->batch());
     std::vector<TrialWork> tw(n);
     for (uint32_t t = 0; t < n; ++t) tw[t] = TrialWork{d_tim, accs[t], mean, sd, 0.0f, 0};
@@ -262,7 +263,8 @@ extern "C" int psx_batch_bound_audit(const psx_search_args* args, const psx_batc
     std::unique_ptr<Engine> eng(new Engine(*args, eo, s));
     PSX_CHECK_HIP(hipMalloc(&d_tim, sizeof(float) * args->size));
     float mean, sd;
-    eng->prologue(d_series, nsamps, d_tim, &mean, &sd, nullptr);
+    eng->set_zap(nullptr, s);
+    eng->prologue(d_series, nsamps, d_tim, &mean, &sd, s);
     const uint32_t n = std::min(naccs, eng->batch());
     std::vector<TrialWork> tw(n);
     for (uint32_t t = 0; t < n; ++t) tw[t] = TrialWork{d_tim, accs[t], mean, sd, 0.0f, 0};
@@ -296,7 +298,6 @@ extern "C" int psx_batch_search(const psx_search_args* args, const psx_batch_opt
   PSX_REQUIRE(!accs || naccs > 0, "psx_batch_search: empty acceleration list");
   hipStream_t s = nullptr, ps = nullptr;
   float* d_tims = nullptr;
-  float* d_stage = nullptr;
   psx::batch::PrologueResult* h_res = nullptr;
   std::vector<hipEvent_t> done_ev;
   auto release = [&]() {
@@ -305,7 +306,6 @@ extern "C" int psx_batch_search(const psx_search_args* args, const psx_batch_opt
       if (e) (void)hipEventDestroy(e);
     if (h_res) (void)hipHostFree(h_res);
     if (d_tims) (void)hipFree(d_tims);
-    if (d_stage) (void)hipFree(d_stage);
     if (ps) (void)hipStreamDestroy(ps);
     if (s) (void)hipStreamDestroy(s);
   };
@@ -338,19 +338,22 @@ extern "C" int psx_batch_search(const psx_search_args* args, const psx_batch_opt
     std::vector<std::vector<float>> acc_lists(ndm);
     AccelerationPlan plan(args->acc_start, args->acc_end, args->acc_tol, args->acc_pulse_width * 1e-6, N,
                           args->tsamp, args->cfreq, args->ch_bw);
-    if (!series_on_device) PSX_CHECK_HIP(hipMalloc(&d_stage, sizeof(float) * nreal));
     std::unique_ptr<Zapper> zap;
     if (args->nbirdies) zap.reset(new Zapper(args->birdie_freq, args->birdie_width, args->nbirdies, ps));
     PSX_CHECK_HIP(hipHostMalloc((void**)&h_res, sizeof(psx::batch::PrologueResult) * ndm, hipHostMallocDefault));
-    done_ev.assign(ndm, nullptr);
+    const uint32_t group = eng->prologue_group();
+    done_ev.assign((ndm + group - 1) / group, nullptr);
     for (auto& e : done_ev) PSX_CHECK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    // every prologue is enqueued at once on ps; the trials of DM d wait for
-    // its event only
+    // the prologues of every group of DMs are enqueued at once on ps; the
+    // trials of a DM wait for its group's event only.  Series in host memory
+    // are uploaded to their place in d_tims first
     auto input_of = [&](uint32_t d, hipStream_t st) {
       const float* src = series + (uint64_t)d * nreal;
       if (series_on_device) return src;
-      hip_check(hipMemcpyAsync(d_stage, src, sizeof(float) * nreal, hipMemcpyHostToDevice, st), "series upload");
-      return (const float*)d_stage;
+      float* tim = d_tims + (uint64_t)d * N;
+      hip_check(hipMemcpyAsync(tim, src, sizeof(float) * std::min<uint64_t>(nreal, N), hipMemcpyHostToDevice, st),
+                "series upload");
+      return (const float*)tim;
     };
     uint64_t ntrials = 0;
     for (uint32_t d = 0; d < ndm; ++d) {
@@ -366,27 +369,33 @@ extern "C" int psx_batch_search(const psx_search_args* args, const psx_batch_opt
     if (ntrials > eng->batch()) eng->prepare((uint32_t)(ntrials % eng->batch()));
     {
       psx::TraceRange dm_range("DM-Loop");  // the per-DM prologues, all queued here
+      eng->set_zap(zap.get(), ps);
+      for (uint32_t d0 = 0; d0 < ndm; d0 += group) {
+        const uint32_t n = std::min(group, ndm - d0);
+        const float* src = input_of(d0, ps);
+        if (!series_on_device)
+          for (uint32_t d = d0 + 1; d < d0 + n; ++d) input_of(d, ps);
+        eng->prologue_async(src, series_on_device ? nreal : N, nreal, d_tims + (uint64_t)d0 * N, n, &h_res[d0], ps);
+        PSX_CHECK_HIP(hipEventRecord(done_ev[d0 / group], ps));
+      }
       for (uint32_t d = 0; d < ndm; ++d) {
-        float* tim = d_tims + (uint64_t)d * N;
-        eng->prologue_async(input_of(d, ps), nreal, tim, &h_res[d], ps, zap.get());
-        PSX_CHECK_HIP(hipEventRecord(done_ev[d], ps));
-        tims[d] = tim;
+        tims[d] = d_tims + (uint64_t)d * N;
         idx[d] = (int)d;
       }
     }
     auto ready = [&](size_t d) {
-      hip_check(hipEventSynchronize(done_ev[d]), "prologue event");
+      const hipEvent_t ev = done_ev[d / group];
+      hip_check(hipEventSynchronize(ev), "prologue event");
       if (!h_res[d].base.done) {
         // the baseline loop needs more than the device steps: redo this DM
-        // with the host-driven prologue once ps is idle (its buffers are
-        // shared), from its original input
+        // with the host-driven loop once ps is idle (the prologue's buffers
+        // are shared), from its original input
         hip_check(hipStreamSynchronize(ps), "prologue stream");
-        eng->prologue(input_of((uint32_t)d, s), nreal, d_tims + d * N, &means[d], &stds[d], zap.get());
-        hip_check(hipStreamSynchronize(s), "prologue");
+        eng->prologue(input_of((uint32_t)d, ps), nreal, d_tims + d * N, &means[d], &stds[d], ps);
       } else {
         eng->stats_of(h_res[d], &means[d], &stds[d]);
       }
-      hip_check(hipStreamWaitEvent(s, done_ev[d], 0), "stream wait");
+      hip_check(hipStreamWaitEvent(s, ev, 0), "stream wait");
     };
     auto t1 = clk::now();
     std::vector<std::vector<Candidate>> per_dm;

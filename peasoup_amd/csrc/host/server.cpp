@@ -72,7 +72,29 @@ struct TrialRef {
   uint32_t acc;
 };
 
+// Pinned memory the prologue results of a request arrive in, grown to the
+// largest request of an engine and freed with it.
+struct PinnedResults {
+  psx::batch::PrologueResult* p = nullptr;
+  uint32_t n = 0;
+  // nothing may be writing the results: the caller's stream is idle
+  void reserve(uint32_t want) {
+    if (want <= n) return;
+    (void)hipHostFree(p);
+    p = nullptr;
+    n = 0;
+    if (hipHostMalloc((void**)&p, want * sizeof(*p), hipHostMallocDefault) != hipSuccess)
+      throw std::runtime_error("pinned allocation failed");
+    n = want;
+  }
+  PinnedResults() = default;
+  ~PinnedResults() { (void)hipHostFree(p); }
+  PinnedResults(const PinnedResults&) = delete;
+  PinnedResults& operator=(const PinnedResults&) = delete;
+};
+
 struct EngineState {
+  PinnedResults res;  // declared first: outlives the engine, whose destructor drains the stream
   std::unique_ptr<Engine> eng;
   hipStream_t stream = nullptr;
   hipEvent_t mark = nullptr;  // the engine stream's work so far (mixed dispatch waits on it)
@@ -326,18 +348,41 @@ bool psx_server::admit_one(Request* r) {
   r->per_trial.resize(ndm);
   AccelerationPlan plan(a.acc_start, a.acc_end, a.acc_tol, a.acc_pulse_width * 1e-6, N, a.tsamp, a.cfreq, a.ch_bw);
   const uint64_t ncopy = std::min<uint64_t>(r->spec.nsamps, N);
-  const hipMemcpyKind kind = r->spec.series_on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
   // every prologue and acceleration list is prepared and checked before any
   // trial of the request is queued, so a request that fails here leaves no
   // work behind
   if (!r->birdie_freq.empty())
     r->zap.reset(new Zapper(r->birdie_freq.data(), r->birdie_width.data(), r->birdie_freq.size(), es->stream));
-  for (uint32_t d = 0; d < ndm; ++d) {
+  // the prologues, in groups, straight from the request's series or from
+  // their upload into the resident buffer
+  Engine& eng = *es->eng;
+  const bool on_dev = r->spec.series_on_device != 0;
+  const uint64_t nsamps = r->spec.nsamps;
+  auto input_of = [&](uint32_t d) {
+    const float* src = r->spec.series + (uint64_t)d * nsamps;
+    if (on_dev) return src;
     float* tim = r->d_tims + (uint64_t)d * N;
-    if (hipMemcpyAsync(tim, r->spec.series + (uint64_t)d * r->spec.nsamps, ncopy * sizeof(float), kind,
-                       es->stream) != hipSuccess)
+    if (hipMemcpyAsync(tim, src, ncopy * sizeof(float), hipMemcpyHostToDevice, es->stream) != hipSuccess)
       throw std::runtime_error("series upload failed");
-    es->eng->prologue(tim, r->spec.nsamps, tim, &r->means[d], &r->stds[d], r->zap.get());
+    return (const float*)tim;
+  };
+  PinnedResults& res = es->res;
+  if (ndm > res.n && hipStreamSynchronize(es->stream) != hipSuccess) throw std::runtime_error("stream failed");
+  res.reserve(ndm);
+  eng.set_zap(r->zap.get(), es->stream);
+  for (uint32_t d0 = 0; d0 < ndm; d0 += eng.prologue_group()) {
+    const uint32_t n = std::min(eng.prologue_group(), ndm - d0);
+    const float* src = input_of(d0);
+    if (!on_dev)
+      for (uint32_t d = d0 + 1; d < d0 + n; ++d) input_of(d);
+    eng.prologue_async(src, on_dev ? nsamps : N, nsamps, r->d_tims + (uint64_t)d0 * N, n, res.p + d0, es->stream);
+  }
+  if (hipStreamSynchronize(es->stream) != hipSuccess) throw std::runtime_error("prologue failed");
+  for (uint32_t d = 0; d < ndm; ++d) {
+    if (res.p[d].base.done)
+      eng.stats_of(res.p[d], &r->means[d], &r->stds[d]);
+    else  // the baseline loop had not stopped on the device
+      eng.prologue(input_of(d), nsamps, r->d_tims + (uint64_t)d * N, &r->means[d], &r->stds[d], es->stream);
     if (!r->accs_override.empty())
       r->acc_lists[d] = r->accs_override;
     else

@@ -12,7 +12,6 @@
 
 #include "common.hpp"
 #include "kernels_dev.hpp"
-#include "reduce_async.hpp"
 #include "trace.hpp"
 
 using psx::as_stream;
@@ -146,19 +145,12 @@ __global__ void __launch_bounds__(kBlock) k_divide(float2* __restrict__ X, const
   }
 }
 
-// zap_birdies_kernel (src/kernels.cu:1063-1084): bins
-// [floor((f-w)/bw), ceil((f+w)/bw)) of each birdie, clamped to [0, nb-1),
-// become 1+0i.  One block per birdie; the bin range is computed in float as
-// the reference does and clamped before any integer conversion.
+// zap_birdies_kernel (src/kernels.cu:1063-1084): each birdie's bins
+// (zap_range) become 1+0i.  One block per birdie.
 __global__ void __launch_bounds__(kBlock) k_zap(float2* __restrict__ X, const float* __restrict__ freqs,
                                                 const float* __restrict__ widths, float bin_width, uint64_t nb) {
-  const float f = freqs[blockIdx.x];
-  const float w = widths[blockIdx.x];
-  const double lo_f = (double)floorf((f - w) / bin_width);
-  const double hi_f = (double)ceilf((f + w) / bin_width);
-  if (!(lo_f < (double)nb)) return;  // also rejects NaN
-  const uint64_t lo = lo_f > 0.0 ? (uint64_t)lo_f : 0;
-  const uint64_t hi = hi_f >= (double)(nb - 1) ? nb - 1 : (hi_f > 0.0 ? (uint64_t)hi_f : 0);
+  uint64_t lo, hi;
+  if (!psx::zap_range(freqs[blockIdx.x], widths[blockIdx.x], bin_width, nb, lo, hi)) return;
   for (uint64_t i = lo + threadIdx.x; i < hi; i += blockDim.x) X[i] = make_float2(1.0f, 0.0f);
 }
 
@@ -167,12 +159,8 @@ __global__ void __launch_bounds__(kBlock) k_zap(float2* __restrict__ X, const fl
 // GPU_rms, src/kernels.cu:433-461, accumulate float terms in float).
 constexpr unsigned kReduceBlocks = 1024;
 
-// skip (optional): a stopped device baseline loop, whose later iterations
-// need no sums.
 __global__ void __launch_bounds__(kBlock) k_sum_sq(const float* __restrict__ x, uint64_t first, uint64_t n,
-                                                   double2* __restrict__ partial,
-                                                   const psx::BaselineState* __restrict__ skip) {
-  if (skip && skip->done) return;
+                                                   double2* __restrict__ partial) {
   double s1 = 0.0, s2 = 0.0;
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t i = first + (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
@@ -196,9 +184,7 @@ __global__ void __launch_bounds__(kBlock) k_sum_sq(const float* __restrict__ x, 
 }
 
 __global__ void __launch_bounds__(kBlock) k_sum_final(const double2* __restrict__ partial, unsigned np,
-                                                      double2* __restrict__ out,
-                                                      const psx::BaselineState* __restrict__ skip) {
-  if (skip && skip->done) return;
+                                                      double2* __restrict__ out) {
   double s1 = 0.0, s2 = 0.0;
   for (unsigned i = threadIdx.x; i < np; i += blockDim.x) {
     s1 += partial[i].x;
@@ -238,33 +224,6 @@ __global__ void __launch_bounds__(kBlock) k_normalise(float* __restrict__ p, uin
 __global__ void __launch_bounds__(kBlock) k_subtract(float* __restrict__ x, uint64_t n, float mean) {
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) x[i] -= mean;
-}
-
-// Device-resident remove_baseline loop (the host loop of
-// psx_remove_baseline with its arithmetic): each step subtracts the mean of
-// the sums in `sums` unless the loop has already stopped, then records
-// whether it continues.
-__global__ void __launch_bounds__(kBlock) k_subtract_dev(float* __restrict__ x, uint64_t n,
-                                                         const double2* __restrict__ sums,
-                                                         const psx::BaselineState* __restrict__ st) {
-  if (st->done) return;
-  const float mean = (float)sums->x / (float)(int64_t)n;
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) x[i] -= mean;
-}
-__global__ void k_baseline_step(uint64_t n, const double2* __restrict__ sums, psx::BaselineState* __restrict__ st) {
-  if (blockIdx.x != 0 || threadIdx.x != 0 || st->done) return;
-  const float mean = (float)sums->x / (float)(int64_t)n;
-  // do { ...; if (count++ > 100) break; } while (fabsf(mean) > 5e-7 * (double)n);
-  const int32_t count = st->count;
-  st->count = count + 1;
-  st->done = (count > 100 || !((double)fabsf(mean) > 5e-7 * (double)n)) ? 1 : 0;
-}
-__global__ void k_baseline_init(psx::BaselineState* st) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    st->count = 0;
-    st->done = 0;
-  }
 }
 
 // GPU_fill (src/kernels.cu:482-488).
@@ -379,11 +338,6 @@ __global__ void k_set_u32(uint32_t* p, uint32_t v) {
   if (blockIdx.x == 0 && threadIdx.x == 0) *p = v;
 }
 
-inline float stretch_step(uint64_t in_count, uint64_t out_count) {
-  // linear_stretch_functor ctor (src/kernels.cu:1015-1016): float / float
-  return (float)(in_count - 1) / (float)(out_count - 1);
-}
-
 }  // namespace
 
 // ============================================================ C ABI
@@ -444,7 +398,7 @@ extern "C" int psx_linear_stretch(const float* in, uint64_t in_count, float* out
   PSX_REQUIRE(in && out && in_count > 0 && out_count > 1, "psx_linear_stretch: bad arguments");
   PSX_REQUIRE(out_count <= 0xFFFFFFFFull, "psx_linear_stretch: out_count exceeds 32-bit index");
   k_stretch<<<psx::grid_for(out_count, kBlock), kBlock, 0, as_stream(s)>>>(in, in_count, out, out_count,
-                                                                           stretch_step(in_count, out_count));
+                                                                           psx::stretch_step(in_count, out_count));
   PSX_CHECK_LAUNCH("k_stretch");
   return psx::ok();
 }
@@ -492,7 +446,7 @@ extern "C" int psx_deredden_median(const float* A, uint64_t nb, double bin_width
   const hipStream_t hs = as_stream(s);
   // zone [0, pos5) <- m5
   if (z1 > z0) {
-    k_stretch_zone<<<psx::grid_for(z1 - z0, kBlock), kBlock, 0, hs>>>(m5, c5, median, z0, z1, stretch_step(c5, nb));
+    k_stretch_zone<<<psx::grid_for(z1 - z0, kBlock), kBlock, 0, hs>>>(m5, c5, median, z0, z1, psx::stretch_step(c5, nb));
     PSX_CHECK_LAUNCH("k_stretch_zone");
   }
   // zone [pos5, pos25) <- m25 (the reference copies pos25 elements from pos5;
@@ -503,14 +457,14 @@ extern "C" int psx_deredden_median(const float* A, uint64_t nb, double bin_width
     const uint64_t hi = z1e < hi25 ? z1e : hi25;
     if (hi > z1) {
       k_stretch_zone<<<psx::grid_for(hi - z1, kBlock), kBlock, 0, hs>>>(m25, c25, median, z1, hi,
-                                                                        stretch_step(c25, nb));
+                                                                        psx::stretch_step(c25, nb));
       PSX_CHECK_LAUNCH("k_stretch_zone");
     }
   }
   // zone [pos25, nb) <- m125
   if (nb > z2) {
     k_stretch_zone<<<psx::grid_for(nb - z2, kBlock), kBlock, 0, hs>>>(m125, c125, median, z2, nb,
-                                                                      stretch_step(c125, nb));
+                                                                      psx::stretch_step(c125, nb));
     PSX_CHECK_LAUNCH("k_stretch_zone");
   }
   return psx::ok();
@@ -569,9 +523,9 @@ static int sum_sq(const float* x, uint64_t first, uint64_t n, void* work, psx_st
   double2* partial = (double2*)work;
   double2* out = partial + kReduceBlocks;
   const unsigned g = psx::grid_for(n - first, kBlock, kReduceBlocks);
-  k_sum_sq<<<g, kBlock, 0, as_stream(s)>>>(x, first, n, partial, nullptr);
+  k_sum_sq<<<g, kBlock, 0, as_stream(s)>>>(x, first, n, partial);
   PSX_CHECK_LAUNCH("k_sum_sq");
-  k_sum_final<<<1, kBlock, 0, as_stream(s)>>>(partial, g, out, nullptr);
+  k_sum_final<<<1, kBlock, 0, as_stream(s)>>>(partial, g, out);
   PSX_CHECK_LAUNCH("k_sum_final");
   double2 h;
   PSX_CHECK_HIP(hipMemcpyAsync(&h, out, sizeof(h), hipMemcpyDeviceToHost, as_stream(s)));
@@ -602,35 +556,6 @@ extern "C" int psx_normalise(float* p, float mean, float sigma, uint64_t n, psx_
   PSX_CHECK_LAUNCH("k_normalise");
   return psx::ok();
 }
-
-namespace psx {
-int sum_sq_async(const float* x, uint64_t first, uint64_t n, void* work, double2* out, hipStream_t s,
-                 const BaselineState* skip) {
-  double2* partial = (double2*)work;
-  const unsigned g = psx::grid_for(n - first, kBlock, kReduceBlocks);
-  k_sum_sq<<<g, kBlock, 0, s>>>(x, first, n, partial, skip);
-  PSX_CHECK_LAUNCH("k_sum_sq");
-  k_sum_final<<<1, kBlock, 0, s>>>(partial, g, out, skip);
-  PSX_CHECK_LAUNCH("k_sum_final");
-  return PSX_OK;
-}
-
-int remove_baseline_async(float* x, uint64_t n, void* work, BaselineState* st, int steps, hipStream_t s) {
-  if (!x || !work || !st || n == 0 || steps < 1) return psx::fail(PSX_ERR_ARG, "remove_baseline_async: bad arguments");
-  double2* sums = (double2*)work + kReduceBlocks;
-  k_baseline_init<<<1, 64, 0, s>>>(st);
-  PSX_CHECK_LAUNCH("k_baseline_init");
-  for (int i = 0; i < steps; ++i) {
-    int rc = sum_sq_async(x, 0, n, work, sums, s, st);
-    if (rc) return rc;
-    k_subtract_dev<<<psx::grid_for(n, kBlock), kBlock, 0, s>>>(x, n, sums, st);
-    PSX_CHECK_LAUNCH("k_subtract_dev");
-    k_baseline_step<<<1, 64, 0, s>>>(n, sums, st);
-    PSX_CHECK_LAUNCH("k_baseline_step");
-  }
-  return PSX_OK;
-}
-}  // namespace psx
 
 // GPU_remove_baseline (src/kernels.cu:463-479).
 extern "C" int psx_remove_baseline(float* x, uint64_t n, void* work, psx_stream s) {

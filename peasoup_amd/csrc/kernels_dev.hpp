@@ -96,6 +96,25 @@ __device__ inline float stretch_at(const float* __restrict__ in, uint64_t in_cou
   return (fr > 1e-5f) ? fmaf(fr, b - a, a) : a + 0.f;
 }
 
+// Step of the stretch of in_count values to out_count
+// (linear_stretch_functor, src/kernels.cu:1015-1016): float / float.
+__host__ __device__ inline float stretch_step(uint64_t in_count, uint64_t out_count) {
+  return (float)(in_count - 1) / (float)(out_count - 1);
+}
+
+// zap_birdies_kernel (src/kernels.cu:1063-1084): bins
+// [floor((f-w)/bw), ceil((f+w)/bw)) of a birdie, clamped to [0, nb-1), as
+// [lo, hi); false when there are none (NaN included).  Computed in float as
+// the reference does and clamped before any integer conversion.
+__device__ inline bool zap_range(float f, float w, float bin_width, uint64_t nb, uint64_t& lo, uint64_t& hi) {
+  const double lo_f = (double)floorf((f - w) / bin_width);
+  const double hi_f = (double)ceilf((f + w) / bin_width);
+  if (!(lo_f < (double)nb)) return false;
+  lo = lo_f > 0.0 ? (uint64_t)lo_f : 0;
+  hi = hi_f >= (double)(nb - 1) ? nb - 1 : (hi_f > 0.0 ? (uint64_t)hi_f : 0);
+  return lo < hi;
+}
+
 // Scale of fold K's running sum (1-based): times 2^-K/2, computed in double
 // for odd K as the reference does (src/kernels.cu:38-98).  Host and device
 // round every step alike (IEEE multiply and conversion, nearest even).

@@ -203,6 +203,8 @@ class Zapper {
                    "Zapper::zap");
   }
   std::size_t size() const { return birdies.size(); }
+  const float* get_device_birdies() const { return d_birdies; }
+  const float* get_device_widths() const { return d_widths; }
   const std::vector<float>& get_birdies() const { return birdies; }
   const std::vector<float>& get_widths() const { return widths; }
 };
