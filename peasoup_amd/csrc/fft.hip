@@ -485,12 +485,40 @@ static bool len_supported(uint64_t L, bool multi) {
   return false;
 }
 
-// Default decomposition: one pass when a single-workgroup kernel exists,
-// else the two-pass split with the longest contiguous (last) pass, whose
-// rows are read and written whole, and the shortest strided pass (measured
-// fastest on MI355X: 1024 x 4096 beats 2048 x 2048 for 2^22 points) while
-// that strided pass is at most 2,048 points, else three passes as below.
-bool default_decomp(uint64_t M, Decomp& d) {
+// Column tiles of a default two-pass plan: 16 columns in the strided pass and
+// 8 rows (16 of at most 256 points) in the last one, where they fit; half as
+// many where that would leave fewer than 192 (strided) or 256 (last)
+// workgroups on the chip's 256 CUs.  Measured, R2C us: 2^21 samples, one
+// transform 30.7 (16 x 4), 26.2 (8 x 4), eight transforms 95.0 / 107.8; 2^22,
+// one transform 40.2 / 37.0, four 98.6 / 112.6; 2^20, one transform,
+// 1,024-point last pass of 4 rows 17.4, of 16 rows 23.5.  Last passes of fewer
+// than 1,024 points keep 8 rows in batched plans: the row-layout kernels of
+// the batched search start there.
+static void two_pass_tiles(Decomp& d, uint32_t batch) {
+  const uint64_t n0 = (uint64_t)d.L[1] / 16 * batch, n1 = (uint64_t)d.L[0] / 8 * batch;
+  const int c0 = n0 >= 192 ? 16 : 8;
+  int c1 = 8;
+  if (d.L[1] <= 256) c1 = n1 / 2 >= 256 ? 16 : 8;
+  else if (n1 < 256 && (batch == 1 || d.L[1] >= 1024)) c1 = 4;
+  const KernelInfo* k0 = find_kernel(d.L[0], c0, PM_COLS_TW, false);
+  const KernelInfo* k1 = find_kernel(d.L[1], c1, PM_ROWS_TO_COLS, false);
+  // a strided pass keeps two workgroups per CU
+  if (k0 && k0->lds <= 80 * 1024) d.C[0] = c0;
+  if (k1 && k1->lds <= 160 * 1024) d.C[1] = c1;
+}
+
+// Default decomposition: one pass when a single-workgroup kernel exists, else
+// two passes of about equal length, the strided one the largest power of two
+// that is at most 1,024 and no longer than the contiguous last one (whose
+// rows are read and written whole).  Against the longest last pass, which
+// this rule replaces below 2^23 samples (R2C of one transform and, in the
+// batched search, us per trial): 2^17 17.2 and 1.68 -> 12.7 and 0.95, 2^20
+// 21.2 and 5.10 -> 17.4 and 5.01, 2^21 31.1 and 10.93 -> 26.3 and 9.80, 3*2^17
+// 27.1 and 4.28 -> 18.6 and 2.22, 3*2^21 65.3 and 36.1 -> 52.8 and 33.2; batched
+// 3*2^20 is even (16.79, 16.87).
+// Longer: the split with the longest last pass while the strided pass is at
+// most 2,048 points (2^24: 2,048 x 4,096), else three passes as below.
+bool default_decomp(uint64_t M, Decomp& d, uint32_t batch) {
   d = Decomp();
   if (!valid_complex_len(M)) return false;
   if (len_supported(M, false)) {
@@ -498,6 +526,16 @@ bool default_decomp(uint64_t M, Decomp& d) {
     d.L[0] = (int)M;
     d.C[0] = 1;
     return true;
+  }
+  for (uint64_t M2 = 1024; M2 >= 32; M2 /= 2) {
+    const uint64_t M1 = M / M2;
+    if (M % M2 || M1 < M2 || M1 > 4096) continue;
+    if (!len_supported(M1, true) || !len_supported(M2, true)) continue;
+    d.npass = 2;
+    d.L[0] = (int)M2;
+    d.L[1] = (int)M1;
+    two_pass_tiles(d, batch);
+    return pick_tiles(d);
   }
   uint64_t bM1 = 0, bM2 = 0;
   for (uint64_t M1 = 32; M1 <= 4096 && M1 < M; M1 = (M1 % 3 == 0) ? (M1 / 3) * 4 : M1 + M1 / 2) {
@@ -818,7 +856,7 @@ int plan_create_with(uint64_t n, int kind, uint32_t batch, const Decomp* forced,
   p->nb = n / 2 + 1;
   p->kind = kind;
   p->batch = batch;
-  bool okd = forced ? (p->d = *forced, pick_tiles(p->d)) : default_decomp(p->M, p->d);
+  bool okd = forced ? (p->d = *forced, pick_tiles(p->d)) : default_decomp(p->M, p->d, batch);
   if (!okd || !decomp_supported(p->d)) {
     delete p;
     return psx::fail(PSX_ERR_UNSUPPORTED, "psx_fft_plan_create: no decomposition for n=%llu",
@@ -1057,7 +1095,7 @@ extern "C" int psx_fft_layout_check(uint64_t n, int kind, uint32_t batch, int np
     }
     okd = psx::fft::pick_tiles(p.d);
   } else {
-    okd = psx::fft::default_decomp(p.M, p.d);
+    okd = psx::fft::default_decomp(p.M, p.d, batch);
   }
   if (!okd || !psx::fft::decomp_supported(p.d)) return psx::fail(PSX_ERR_UNSUPPORTED, "no decomposition");
   uint64_t prod = 1;

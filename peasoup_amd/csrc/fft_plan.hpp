@@ -21,7 +21,8 @@ struct Decomp {
 };
 
 bool valid_complex_len(uint64_t m);
-bool default_decomp(uint64_t M, Decomp& d);
+// batch: transforms per launch (sets the column tiles, not the lengths).
+bool default_decomp(uint64_t M, Decomp& d, uint32_t batch);
 bool pick_tiles(Decomp& d);
 bool decomp_supported(const Decomp& d);
 // Roots W_n^k of the real length n as a two-level table: W = hi[k>>shift]*lo[k&mask].
