@@ -444,27 +444,27 @@ int configure_lds() {
   return PSX_OK;
 }
 
-// ------------------------------------------------------- host tables
-void root_table_host(uint64_t m, uint32_t shift, std::vector<float2>& lo, std::vector<float2>& hi) {
-  // W_m^x = W_m^(hi part) * W_m^(lo part), x = (h << shift) + l
-  const uint64_t T = 1ull << shift;
-  lo.resize(T);
-  hi.resize((m + T - 1) / T + 1);
-  const long double tp = -2.0L * 3.14159265358979323846264338327950288L / (long double)m;
-  for (uint64_t l = 0; l < T; ++l) {
-    long double a = tp * (long double)l;
-    lo[l] = make_float2((float)cosl(a), (float)sinl(a));
+// ------------------------------------------------------- root tables
+// One run of a plan's tables: entry i holds W_mod^(i*step).
+struct RootRun {
+  uint64_t at, count, step, mod;
+};
+constexpr int kMaxRuns = 16;
+struct RootRuns {
+  RootRun r[kMaxRuns];
+  int n;
+};
+// All tables of a plan in one launch, in double (the host's long double
+// cosl/sinl took 6.5 ms for a 2^23-sample plan; this and the allocations take
+// 0.05 ms).
+__global__ void __launch_bounds__(256) k_roots(float2* __restrict__ tables, const RootRuns runs) {
+  const RootRun run = runs.r[blockIdx.y];
+  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < run.count; i += stride) {
+    double s, c;
+    sincospi(-2.0 * (double)(i * run.step) / (double)run.mod, &s, &c);
+    tables[run.at + i] = make_float2((float)c, (float)s);
   }
-  for (uint64_t h = 0; h < hi.size(); ++h) {
-    long double a = tp * (long double)(h * T);
-    hi[h] = make_float2((float)cosl(a), (float)sinl(a));
-  }
-}
-
-void twl_host(int L, std::vector<float2>& t) {
-  t.resize(L);
-  const long double tp = -2.0L * 3.14159265358979323846264338327950288L / (long double)L;
-  for (int e = 0; e < L; ++e) t[e] = make_float2((float)cosl(tp * e), (float)sinl(tp * e));
 }
 
 }  // namespace
@@ -688,16 +688,25 @@ int build_passes(psx_fft_plan* p, bool device_tables) {
   const Decomp& d = p->d;
   const uint64_t M = p->M;
   // --- device tables: per-pass W_L, four-step roots, W_n roots
-  std::vector<float2> host;
-  std::vector<size_t> twl_off(d.npass), tw4lo_off(d.npass), tw4hi_off(d.npass), tw4r_off(d.npass);
-  std::vector<uint32_t> tw4_shift(d.npass);
-  auto append = [&](const std::vector<float2>& v) {
-    size_t o = host.size();
-    host.insert(host.end(), v.begin(), v.end());
-    while (host.size() % 32) host.push_back(make_float2(0.f, 0.f));
+  RootRuns runs{};
+  size_t size = 0;
+  size_t twl_off[3] = {}, tw4lo_off[3] = {}, tw4hi_off[3] = {}, tw4r_off[3] = {};
+  uint32_t tw4_shift[3] = {};
+  auto append = [&](uint64_t count, uint64_t step, uint64_t mod) {
+    const size_t o = size;
+    runs.r[runs.n++] = RootRun{o, count, step, mod};
+    size = (o + count + 31) / 32 * 32;
     return o;
   };
-  std::vector<float2> tmp, lo, hi;
+  // W_m^x = W_m^(hi part) * W_m^(lo part), x = (h << shift) + l, the two
+  // tables about equally long
+  auto append_two = [&](uint64_t m, uint32_t& shift, size_t& lo, size_t& hi) {
+    shift = 0;
+    while ((1ull << (shift + 1)) * (1ull << (shift + 1)) <= m && (m % (1ull << (shift + 1))) == 0) ++shift;
+    const uint64_t T = 1ull << shift;
+    lo = append(T, 1, m);
+    hi = append((m + T - 1) / T + 1, T, m);
+  };
   // four-step twiddle sizes per pass
   uint64_t mtw[3] = {0, 0, 0};
   if (d.npass == 2) mtw[0] = M;
@@ -705,34 +714,27 @@ int build_passes(psx_fft_plan* p, bool device_tables) {
     mtw[0] = M;
     mtw[1] = (uint64_t)d.L[1] * (uint64_t)d.L[2];
   }
+  static_assert(3 + 2 * 3 + 2 <= kMaxRuns, "runs of a three-pass plan");
   for (int q = 0; q < d.npass; ++q) {
-    twl_host(d.L[q], tmp);
-    twl_off[q] = append(tmp);
+    twl_off[q] = append((uint64_t)d.L[q], 1, (uint64_t)d.L[q]);
     if (mtw[q]) {
-      uint32_t sh = 0;
-      while ((1ull << (sh + 1)) * (1ull << (sh + 1)) <= mtw[q] && (mtw[q] % (1ull << (sh + 1))) == 0) ++sh;
-      tw4_shift[q] = sh;
-      root_table_host(mtw[q], sh, lo, hi);
-      tw4lo_off[q] = append(lo);
-      tw4hi_off[q] = append(hi);
+      append_two(mtw[q], tw4_shift[q], tw4lo_off[q], tw4hi_off[q]);
       // W_T^k, T = Mtw * R / L with R the pass's last radix (the output
       // twiddle's column factor)
       const uint64_t T = mtw[q] * (uint64_t)psx::fft::radix_at(d.L[q], psx::fft::num_stages(d.L[q]) - 1) /
                          (uint64_t)d.L[q];
-      tmp.resize(T);
-      const long double tpr = -2.0L * 3.14159265358979323846264338327950288L / (long double)T;
-      for (uint64_t k = 0; k < T; ++k) tmp[k] = make_float2((float)cosl(tpr * k), (float)sinl(tpr * k));
-      tw4r_off[q] = append(tmp);
+      tw4r_off[q] = append(T, 1, T);
     }
   }
   uint32_t rsh = 0;
-  const uint64_t n = p->n;
-  while ((1ull << (rsh + 1)) * (1ull << (rsh + 1)) <= n && (n % (1ull << (rsh + 1))) == 0) ++rsh;
-  root_table_host(n, rsh, lo, hi);
-  const size_t rlo = append(lo), rhi = append(hi);
+  size_t rlo = 0, rhi = 0;
+  append_two(p->n, rsh, rlo, rhi);
   if (device_tables) {
-    PSX_CHECK_HIP(hipMalloc(&p->tables, host.size() * sizeof(float2)));
-    PSX_CHECK_HIP(hipMemcpy(p->tables, host.data(), host.size() * sizeof(float2), hipMemcpyHostToDevice));
+    PSX_CHECK_HIP(hipMalloc(&p->tables, size * sizeof(float2)));
+    k_roots<<<dim3(64, runs.n), 256>>>(p->tables, runs);
+    PSX_CHECK_LAUNCH("k_roots");
+    // plans run on any stream
+    PSX_CHECK_HIP(hipStreamSynchronize(nullptr));
   }
   p->rt = RootTable{p->tables + rlo, p->tables + rhi, rsh, (uint32_t)((1ull << rsh) - 1)};
 
