@@ -461,49 +461,12 @@ __global__ void __launch_bounds__(kB) k_spec_rows(const float2* __restrict__ Y, 
 // to `out` with one atomic per bin row of a wave (all folds together); the
 // host orders them by bin.
 //
-// A wave covers kHarmWaveBins consecutive bins; lane l holds the D bins
-// base + l + 64d.  Fold k's harmonic j of bin i is bin (j*i + 2^(k-1)) >> k,
-// and with i = i0 + 64d that is ((j*i0 + 2^(k-1)) >> k) + d*64j/2^k exactly
-// (2^k divides 64), so each harmonic costs one index per lane and D loads at
-// constant instruction offsets from it: the gathers stay coalesced across
-// lanes and the index arithmetic of harmonic_sums32 drops out of the loop.
-// The running sums take the same addends in the same order as
-// harmonic_sums32, so the thresholded values are bit-identical to it.  The
+// A wave covers kHarmWaveBins consecutive bins, D per lane, through
+// add_harmonic (kernels_dev.hpp): the running sums take harmonic_sums32's
+// addends in its order, so the thresholded values are bit-identical to it.  The
 // loop only decides whether any value of a lane crosses the threshold; a
 // wave with a crossing recomputes its bins one by one with harmonic_sums32,
 // applies the fold windows and appends.
-//
-// Harmonics at 1/16 of the bin or less (step <= 4) touch only D*step + 1
-// consecutive bins per wave, fewer than 64: the wave loads them once (one
-// load per lane) and each d takes its value from the owning lane with
-// ds_bpermute, instead of D loads of a few distinct floats each (2% faster
-// harmonic pass).  The values are the same bins, so the sums are unchanged.
-template <int K, int J, int D>
-__device__ inline void add_harmonic(const PSX_GLOBAL float* p, uint32_t i0, float (&val)[D]) {
-  constexpr uint32_t step = (64u * J) >> K;
-  constexpr uint32_t c = 1u << (K - 1);
-  if constexpr (step <= 4 && D * step + 1 < 64) {
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t s0 = (J * (i0 - lane) + c) >> K;  // the wave's first bin of this harmonic
-    const uint32_t r = ((J * i0 + c) >> K) - s0;     // this lane's offset, <= step
-    const float chunk = p[s0 + lane];
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-      const int addr = (int)((r + (uint32_t)d * step) << 2);
-      val[d] += __int_as_float(__builtin_amdgcn_ds_bpermute(addr, __float_as_int(chunk)));
-    }
-  } else {
-    const PSX_GLOBAL float* q = p + ((J * i0 + c) >> K);
-#pragma unroll
-    for (int d = 0; d < D; ++d) val[d] += q[d * step];
-  }
-}
-// odd harmonics J, J+2, ... below JEND of fold K, in increasing order
-template <int K, int J, int JEND, int D>
-__device__ inline void add_harmonics(const PSX_GLOBAL float* p, uint32_t i0, float (&val)[D]) {
-  add_harmonic<K, J, D>(p, i0, val);
-  if constexpr (J + 2 < JEND) add_harmonics<K, J + 2, JEND, D>(p, i0, val);
-}
 template <int K, int D>
 __device__ inline bool fold_crosses(const float (&val)[D], float thr) {
   bool any = false;
@@ -536,24 +499,24 @@ __global__ void __launch_bounds__(kB) k_harm_peaks(const float* __restrict__ P, 
       for (int d = 0; d < D; ++d) any |= val[d] > w.thr;
     }
     if constexpr (NF > 0) {
-      add_harmonic<1, 1, D>(pg, i0, val);
+      psx::add_harmonic<1, 1, D>(pg, i0, val);
       any |= fold_crosses<1, D>(val, w.thr);
     }
     if constexpr (NF > 1) {
-      add_harmonic<2, 3, D>(pg, i0, val);  // 3/4 before 1/4, as the reference
-      add_harmonic<2, 1, D>(pg, i0, val);
+      psx::add_harmonic<2, 3, D>(pg, i0, val);  // 3/4 before 1/4, as the reference
+      psx::add_harmonic<2, 1, D>(pg, i0, val);
       any |= fold_crosses<2, D>(val, w.thr);
     }
     if constexpr (NF > 2) {
-      add_harmonics<3, 1, 8, D>(pg, i0, val);
+      psx::add_harmonics<3, 1, 8, D>(pg, i0, val);
       any |= fold_crosses<3, D>(val, w.thr);
     }
     if constexpr (NF > 3) {
-      add_harmonics<4, 1, 16, D>(pg, i0, val);
+      psx::add_harmonics<4, 1, 16, D>(pg, i0, val);
       any |= fold_crosses<4, D>(val, w.thr);
     }
     if constexpr (NF > 4) {
-      add_harmonics<5, 1, 32, D>(pg, i0, val);
+      psx::add_harmonics<5, 1, 32, D>(pg, i0, val);
       any |= fold_crosses<5, D>(val, w.thr);
     }
     // survivors are rare: one ballot decides whether this wave appends at all

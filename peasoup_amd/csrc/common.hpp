@@ -7,6 +7,11 @@
 
 #include "psx.h"
 
+// The global address space: accesses through it are global_load/store rather
+// than flat ones.  Global memory takes any alignment on gfx950, so vector
+// types with a smaller alignment attribute are still one instruction.
+#define PSX_GLOBAL __attribute__((address_space(1)))
+
 namespace psx {
 
 // Records a thread-local error message and returns code.

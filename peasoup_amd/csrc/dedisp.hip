@@ -26,8 +26,6 @@ namespace {
 constexpr unsigned kB = 256;
 constexpr uint32_t kMaxChans = 8192;
 
-// Unaligned accesses: global memory takes any byte address on gfx950.
-#define PSX_GLOBAL __attribute__((address_space(1)))
 typedef uint32_t psx_u1 __attribute__((ext_vector_type(1), aligned(1)));
 typedef uint32_t psx_u4 __attribute__((ext_vector_type(4), aligned(1)));
 typedef float psx_f4 __attribute__((ext_vector_type(4), aligned(4)));

@@ -15,6 +15,8 @@
 
 #include <cstdint>
 
+#include "common.hpp"
+
 namespace psx {
 namespace fft {
 
@@ -112,7 +114,6 @@ __host__ __device__ constexpr int pass_lds_bytes(int L, int C, int mode) {
 // 64-bit address arithmetic (generic pointers otherwise become flat
 // accesses with 64-bit VGPR addresses).  Offsets stay below 2^32 bytes: an
 // index is below n <= 2^28 samples.
-#define PSX_GLOBAL __attribute__((address_space(1)))
 typedef float psx_f2v __attribute__((ext_vector_type(2)));
 
 __device__ inline float2 ldg2(const float2* base, uint32_t i) {

@@ -7,6 +7,7 @@
 // to keep every CU busy.  Device code is compiled with -ffp-contract=off; the
 // multiply-adds that the reference's nvcc build contracts are written as
 // explicit fma so that results match the CPU restatement bit for bit.
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 
@@ -118,14 +119,57 @@ __global__ void __launch_bounds__(kBlock) k_stretch(const float* __restrict__ in
     out[i] = psx::stretch_at(in, in_count, (unsigned)i, step);
 }
 
-// Dereddener::calculate_median zone copy (dereddener.hpp:53-61): writes the
-// stretched median of zone z into median[lo, hi).
-__global__ void __launch_bounds__(kBlock) k_stretch_zone(const float* __restrict__ in, uint64_t in_count,
-                                                         float* __restrict__ out, uint64_t lo, uint64_t hi,
-                                                         float step) {
+// The three scrunches of Dereddener::calculate_median (dereddener.hpp:41-52)
+// in one launch: a workgroup stages 125 * kM125 bins in LDS and scrunches them
+// to 5, 25 and 125 bins (2^21 bins: 5.8 us, three launches 8.3 us and their
+// gaps).
+constexpr uint32_t kM125 = 16;
+
+__global__ void __launch_bounds__(kBlock) k_scrunch125(const float* __restrict__ in, float* __restrict__ m5,
+                                                       float* __restrict__ m25, float* __restrict__ m125, uint64_t c5,
+                                                       uint64_t c25, uint64_t c125) {
+  __shared__ float a[125 * kM125], s5[25 * kM125], s25[5 * kM125];
+  const uint64_t b = blockIdx.x;
+  const float* p = in + b * 125 * kM125;
+  const uint64_t left = 5 * c5 - b * 125 * kM125;
+#pragma unroll
+  for (uint32_t i = threadIdx.x; i < 125 * kM125; i += kBlock) a[i] = i < left ? p[i] : 0.f;
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < 25 * kM125; i += kBlock) {
+    const float* q = a + 5 * i;
+    s5[i] = psx::median5(q[0], q[1], q[2], q[3], q[4]);
+    if (b * 25 * kM125 + i < c5) m5[b * 25 * kM125 + i] = s5[i];
+  }
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < 5 * kM125; i += kBlock) {
+    const float* q = s5 + 5 * i;
+    s25[i] = psx::median5(q[0], q[1], q[2], q[3], q[4]);
+    if (b * 5 * kM125 + i < c25) m25[b * 5 * kM125 + i] = s25[i];
+  }
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < kM125; i += kBlock) {
+    const float* q = s25 + 5 * i;
+    if (b * kM125 + i < c125) m125[b * kM125 + i] = psx::median5(q[0], q[1], q[2], q[3], q[4]);
+  }
+}
+
+// Dereddener::calculate_median zone copies (dereddener.hpp:53-61) in one
+// launch: the third zone, from z2, overwrites the others, the first ends at
+// z1, the second at hi; bins of no zone are left as they are.
+struct Stretch {
+  const float* in;
+  uint64_t count;
+  float step;
+};
+__global__ void __launch_bounds__(kBlock) k_stretch_zones(Stretch s5, Stretch s25, Stretch s125, uint64_t z1,
+                                                          uint64_t hi, uint64_t z2, float* __restrict__ out,
+                                                          uint64_t nb) {
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t i = lo + (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < hi; i += stride)
-    out[i] = psx::stretch_at(in, in_count, (unsigned)i, step);
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nb; i += stride) {
+    const Stretch& s = i >= z2 ? s125 : (i < z1 ? s5 : s25);
+    if (i < z2 && i >= z1 && i >= hi) continue;
+    out[i] = psx::stretch_at(s.in, s.count, (unsigned)i, s.step);
+  }
 }
 
 // divide_c_by_f_kernel (src/kernels.cu:1040-1049).
@@ -159,49 +203,57 @@ __global__ void __launch_bounds__(kBlock) k_zap(float2* __restrict__ X, const fl
 // GPU_rms, src/kernels.cu:433-461, accumulate float terms in float).
 constexpr unsigned kReduceBlocks = 1024;
 
+// The workgroup's sums in thread 0: halving tree, its first two levels
+// through LDS and the rest inside wave 0.
+__device__ inline double2 block_sum2(double s1, double s2) {
+  __shared__ double r1[kBlock], r2[kBlock];
+  const unsigned t = threadIdx.x;
+  r1[t] = s1;
+  r2[t] = s2;
+  __syncthreads();
+  if (t < 64) {
+    static_assert(kBlock == 256, "two LDS levels");
+    s1 = (r1[t] + r1[t + 128]) + (r1[t + 64] + r1[t + 192]);
+    s2 = (r2[t] + r2[t + 128]) + (r2[t + 64] + r2[t + 192]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      s1 += __shfl_down(s1, o);
+      s2 += __shfl_down(s2, o);
+    }
+  }
+  return make_double2(s1, s2);
+}
+
 __global__ void __launch_bounds__(kBlock) k_sum_sq(const float* __restrict__ x, uint64_t first, uint64_t n,
                                                    double2* __restrict__ partial) {
   double s1 = 0.0, s2 = 0.0;
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+#pragma unroll 8
   for (uint64_t i = first + (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
     const float v = x[i];
     const float sq = v * v;
     s1 += (double)v;
     s2 += (double)sq;
   }
-  __shared__ double r1[kBlock], r2[kBlock];
-  r1[threadIdx.x] = s1;
-  r2[threadIdx.x] = s2;
-  __syncthreads();
-  for (unsigned o = kBlock / 2; o > 0; o >>= 1) {
-    if (threadIdx.x < o) {
-      r1[threadIdx.x] += r1[threadIdx.x + o];
-      r2[threadIdx.x] += r2[threadIdx.x + o];
-    }
-    __syncthreads();
+  const double2 s = block_sum2(s1, s2);
+  if (threadIdx.x == 0) partial[blockIdx.x] = s;
+}
+
+// The partial sums' total, in thread 0 of the calling workgroup.
+__device__ inline double2 sum_partials(const double2* __restrict__ partial, unsigned np) {
+  double s1 = 0.0, s2 = 0.0;
+#pragma unroll 4
+  for (unsigned i = threadIdx.x; i < np; i += kBlock) {
+    s1 += partial[i].x;
+    s2 += partial[i].y;
   }
-  if (threadIdx.x == 0) partial[blockIdx.x] = make_double2(r1[0], r2[0]);
+  return block_sum2(s1, s2);
 }
 
 __global__ void __launch_bounds__(kBlock) k_sum_final(const double2* __restrict__ partial, unsigned np,
                                                       double2* __restrict__ out) {
-  double s1 = 0.0, s2 = 0.0;
-  for (unsigned i = threadIdx.x; i < np; i += blockDim.x) {
-    s1 += partial[i].x;
-    s2 += partial[i].y;
-  }
-  __shared__ double r1[kBlock], r2[kBlock];
-  r1[threadIdx.x] = s1;
-  r2[threadIdx.x] = s2;
-  __syncthreads();
-  for (unsigned o = kBlock / 2; o > 0; o >>= 1) {
-    if (threadIdx.x < o) {
-      r1[threadIdx.x] += r1[threadIdx.x + o];
-      r2[threadIdx.x] += r2[threadIdx.x + o];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[0] = make_double2(r1[0], r2[0]);
+  const double2 s = sum_partials(partial, np);
+  if (threadIdx.x == 0) out[0] = s;
 }
 
 // normalisation_kernel (src/kernels.cu:496-507).
@@ -220,9 +272,55 @@ __global__ void __launch_bounds__(kBlock) k_normalise(float* __restrict__ p, uin
     p[i] = (p[i] - mean) / sigma;
 }
 
-// GPU_remove_baseline body (src/kernels.cu:471-473): x -= mean.
-__global__ void __launch_bounds__(kBlock) k_subtract(float* __restrict__ x, uint64_t n, float mean) {
+// GPU_remove_baseline (src/kernels.cu:463-479) without a host round trip per
+// iteration:
+//   do { mean; x -= mean; if (count++ > 100) break; } while (fabsf(mean) > 5e-7 * (double)n);
+// k_base_sum's partial sums are totalled by every workgroup of k_base_sub,
+// which subtracts; its first one keeps the loop's state.  Once the loop has
+// stopped, later iterations do nothing.  FIRST: the state is not read.
+struct BaselineState {
+  int32_t count;
+  int32_t done;
+};
+template <bool FIRST>
+__global__ void __launch_bounds__(kBlock) k_base_sum(const float* __restrict__ x, uint64_t n,
+                                                     double2* __restrict__ partial,
+                                                     const BaselineState* __restrict__ st) {
+  if (!FIRST && st->done) return;
+  double s = 0.0;
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+#pragma unroll 8
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) s += (double)x[i];
+  s = block_sum2(s, 0.0).x;
+  if (threadIdx.x == 0) partial[blockIdx.x].x = s;
+}
+// prev, next: the state before and after this iteration, in different places
+// (workgroups that start late still read the one before).
+template <bool FIRST>
+__global__ void __launch_bounds__(kBlock) k_base_sub(float* __restrict__ x, uint64_t n,
+                                                     const double2* __restrict__ partial, unsigned np,
+                                                     const BaselineState* __restrict__ prev,
+                                                     BaselineState* __restrict__ next) {
+  BaselineState st{0, 0};
+  if constexpr (!FIRST) {
+    st = *prev;
+    if (st.done) {
+      if (blockIdx.x == 0 && threadIdx.x == 0) *next = st;
+      return;
+    }
+  }
+  __shared__ float shared_mean;
+  const double s = sum_partials(partial, np).x;
+  if (threadIdx.x == 0) {
+    const float mean = (float)s / (float)(int64_t)n;
+    shared_mean = mean;
+    if (blockIdx.x == 0)
+      *next = BaselineState{st.count + 1, (st.count > 100 || !((double)fabsf(mean) > 5e-7 * (double)n)) ? 1 : 0};
+  }
+  __syncthreads();
+  const float mean = shared_mean;
+  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+#pragma unroll 4
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) x[i] -= mean;
 }
 
@@ -246,8 +344,66 @@ struct FoldPtrs {
   float* f[5];
 };
 
+// Stores fold K of the lane's bins.
+template <int K, int D>
+__device__ inline void store_fold(float* __restrict__ f, uint32_t i0, const float (&val)[D]) {
+  PSX_GLOBAL float* q = (PSX_GLOBAL float*)f + i0;
+#pragma unroll
+  for (int d = 0; d < D; ++d) q[64 * d] = psx::fold_scale<K>(val[d]);
+}
+
+// A wave takes 64 * D consecutive bins through add_harmonic (nb <= 2^27);
+// the last, partial stretch goes bin by bin.  Bound by the traffic behind the
+// L2s: the folds' spans re-read the spectrum 8.5 times for four folds (each
+// XCD's 4 MB L2 holds a quarter of 2^22 + 1 bins) beside the 67 MB written.
+// 2^22 + 1 bins, four folds: 30.3 us with one bin per thread (64-bit indices),
+// 25.7 us here with 2, 4 or 8 bins per lane; 2^19 + 1 bins, 5.6 us and 3.9
+// (4.3 with 8 per lane).
+constexpr int kHarmD = 4;
 template <int NF>
-__global__ void __launch_bounds__(kBlock) k_harmonic(const float* __restrict__ P, FoldPtrs folds, uint64_t nb) {
+__global__ void __launch_bounds__(kBlock) k_harmonic(const float* __restrict__ P, FoldPtrs folds, uint32_t nb) {
+  constexpr uint32_t kWave = 64 * kHarmD;
+  const PSX_GLOBAL float* p = (const PSX_GLOBAL float*)P;
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t base = (blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * kWave;
+  if (base >= nb) return;
+  const uint32_t i0 = base + lane;
+  if (base + kWave > nb) {
+    for (uint32_t i = i0; i < nb; i += 64) {
+      float s[5];
+      psx::harmonic_sums32<NF>(P, i, s);
+#pragma unroll
+      for (int k = 0; k < NF; ++k) folds.f[k][i] = s[k];
+    }
+    return;
+  }
+  float val[kHarmD];
+#pragma unroll
+  for (int d = 0; d < kHarmD; ++d) val[d] = p[i0 + 64 * d];
+  psx::add_harmonic<1, 1, kHarmD>(p, i0, val);
+  store_fold<1>(folds.f[0], i0, val);
+  if constexpr (NF > 1) {
+    psx::add_harmonic<2, 3, kHarmD>(p, i0, val);  // 3/4 before 1/4, as the reference
+    psx::add_harmonic<2, 1, kHarmD>(p, i0, val);
+    store_fold<2>(folds.f[1], i0, val);
+  }
+  if constexpr (NF > 2) {
+    psx::add_harmonics<3, 1, 8, kHarmD>(p, i0, val);
+    store_fold<3>(folds.f[2], i0, val);
+  }
+  if constexpr (NF > 3) {
+    psx::add_harmonics<4, 1, 16, kHarmD>(p, i0, val);
+    store_fold<4>(folds.f[3], i0, val);
+  }
+  if constexpr (NF > 4) {
+    psx::add_harmonics<5, 1, 32, kHarmD>(p, i0, val);
+    store_fold<5>(folds.f[4], i0, val);
+  }
+}
+
+// Spectra of more than 2^27 bins: 64-bit indices, one bin per thread.
+template <int NF>
+__global__ void __launch_bounds__(kBlock) k_harmonic_long(const float* __restrict__ P, FoldPtrs folds, uint64_t nb) {
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nb; i += stride) {
     float s[5];
@@ -257,30 +413,64 @@ __global__ void __launch_bounds__(kBlock) k_harmonic(const float* __restrict__ P
   }
 }
 
+template <int NF>
+void launch_harmonic(const float* P, const FoldPtrs& fp, uint64_t nb, hipStream_t s) {
+  if (nb <= (1ull << 27)) {
+    const uint64_t per = 64 * kHarmD * (kBlock / 64);
+    k_harmonic<NF><<<(unsigned)((nb + per - 1) / per), kBlock, 0, s>>>(P, fp, (uint32_t)nb);
+  } else {
+    k_harmonic_long<NF><<<psx::grid_for(nb, kBlock), kBlock, 0, s>>>(P, fp, nb);
+  }
+}
+
 // ------------------------------------------------------------- peak finding
 // device_find_peaks (src/kernels.cu:391-423) as a two-kernel ordered
-// compaction: per-tile counts, then each tile sums the counts of the tiles
-// before it and writes its survivors in index order using wave ballots and
-// mbcnt prefix sums.
+// compaction: per-tile counts, then each tile with survivors sums the counts
+// of the tiles before it and writes them in index order (the last tile does
+// so for the total).  Survivors are rare: the counting pass streams (16 bins
+// per thread, all four loads in flight), and almost every workgroup of the
+// writing pass ends at its count.  4.2 M bins: 7.1 + 8.3 us (one bin per load,
+// every workgroup summing counts) -> 4.8 + 4.1 us.
 constexpr unsigned kPeakTile = kBlock * 16;
+typedef float psx_f4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// Bins 4*(thread + kBlock*r) .. + 3 of a tile that ends at bin n (< 4: some).
+__device__ inline void peak_load(const float* tile, int64_t n, unsigned r, float thr, float (&v)[4], bool (&hit)[4]) {
+  const int64_t at = 4 * (int64_t)(threadIdx.x + kBlock * r);
+  if (at + 4 <= n) {
+    const psx_f4u x = *(const PSX_GLOBAL psx_f4u*)((const PSX_GLOBAL float*)tile + at);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = x[j];
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = at + j < n ? tile[at + j] : thr;
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) hit[j] = at + j < n && v[j] > thr;
+}
 
 __global__ void __launch_bounds__(kBlock) k_peak_count(const float* __restrict__ p, int64_t start, int64_t end,
                                                        float thr, uint32_t* __restrict__ counts) {
   const int64_t base = start + (int64_t)blockIdx.x * kPeakTile;
+  const int64_t n = min(end - base, (int64_t)kPeakTile);
   unsigned c = 0;
-#pragma unroll 4
-  for (unsigned r = 0; r < kPeakTile / kBlock; ++r) {
-    const int64_t i = base + (int64_t)r * kBlock + threadIdx.x;
-    if (i < end && p[i] > thr) ++c;
+#pragma unroll
+  for (unsigned r = 0; r < kPeakTile / (4 * kBlock); ++r) {
+    float v[4];
+    bool hit[4];
+    peak_load(p + base, n, r, thr, v, hit);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c += (unsigned)__popcll(__ballot(hit[j]));
   }
-  __shared__ unsigned red[kBlock];
-  red[threadIdx.x] = c;
+  __shared__ unsigned wave_cnt[kBlock / 64];
+  if ((threadIdx.x & 63u) == 0) wave_cnt[threadIdx.x >> 6] = c;
   __syncthreads();
-  for (unsigned o = kBlock / 2; o > 0; o >>= 1) {
-    if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-    __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned sum = 0;
+#pragma unroll
+    for (unsigned w = 0; w < kBlock / 64; ++w) sum += wave_cnt[w];
+    counts[blockIdx.x] = sum;
   }
-  if (threadIdx.x == 0) counts[blockIdx.x] = red[0];
 }
 
 __global__ void __launch_bounds__(kBlock) k_peak_write(const float* __restrict__ p, int64_t start, int64_t end,
@@ -288,49 +478,56 @@ __global__ void __launch_bounds__(kBlock) k_peak_write(const float* __restrict__
                                                        unsigned ntiles, int32_t* __restrict__ oidx,
                                                        float* __restrict__ osnr, uint32_t cap,
                                                        uint32_t* __restrict__ total) {
-  __shared__ unsigned red[kBlock];
-  __shared__ unsigned wave_cnt[kBlock / 64];
-  // exclusive prefix of the tile counts before this tile
-  unsigned pre = 0;
-  for (unsigned t = threadIdx.x; t < blockIdx.x; t += kBlock) pre += counts[t];
-  red[threadIdx.x] = pre;
-  __syncthreads();
-  for (unsigned o = kBlock / 2; o > 0; o >>= 1) {
-    if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-    __syncthreads();
-  }
-  unsigned offset = red[0];
   const unsigned mine = counts[blockIdx.x];
-  if (blockIdx.x == ntiles - 1 && threadIdx.x == 0) *total = offset + mine;
-  if (mine == 0) return;
+  const bool last = blockIdx.x == ntiles - 1;
+  if (mine == 0 && !last) return;
+  __shared__ unsigned wave_cnt[kBlock / 64];
   const unsigned lane = threadIdx.x & 63u;
   const unsigned wave = threadIdx.x >> 6;
+  // survivors of the tiles before this one
+  unsigned pre = 0;
+  for (unsigned t = threadIdx.x; t < blockIdx.x; t += kBlock) pre += counts[t];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) pre += __shfl_down(pre, o);
+  if (lane == 0) wave_cnt[wave] = pre;
+  __syncthreads();
+  unsigned offset = 0;
+#pragma unroll
+  for (unsigned w = 0; w < kBlock / 64; ++w) offset += wave_cnt[w];
+  if (last && threadIdx.x == 0) *total = offset + mine;
+  if (mine == 0) return;
   const int64_t base = start + (int64_t)blockIdx.x * kPeakTile;
-  for (unsigned r = 0; r < kPeakTile / kBlock; ++r) {
-    const int64_t i = base + (int64_t)r * kBlock + threadIdx.x;
-    float v = 0.f;
-    bool hit = false;
-    if (i < end) {
-      v = p[i];
-      hit = v > thr;
+  const int64_t n = min(end - base, (int64_t)kPeakTile);
+  for (unsigned r = 0; r < kPeakTile / (4 * kBlock); ++r) {
+    float v[4];
+    bool hit[4];
+    peak_load(p + base, n, r, thr, v, hit);
+    uint64_t mask[4];
+    unsigned before = 0, wave_n = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      mask[j] = __ballot(hit[j]);
+      before += psx::mbcnt64(mask[j]);  // the lower lanes' survivors
+      wave_n += (unsigned)__popcll(mask[j]);
     }
-    const unsigned n_round = __syncthreads_count(hit);
-    if (n_round == 0) continue;
-    const uint64_t mask = __ballot(hit);
-    const unsigned lane_pre = psx::mbcnt64(mask);
-    if (lane == 0) wave_cnt[wave] = (unsigned)__popcll(mask);
     __syncthreads();
-    unsigned wpre = 0;
-    for (unsigned w = 0; w < wave; ++w) wpre += wave_cnt[w];
-    if (hit) {
-      const unsigned pos = offset + wpre + lane_pre;
-      if (pos < cap) {
-        oidx[pos] = (int32_t)i;
-        osnr[pos] = v;
+    if (lane == 0) wave_cnt[wave] = wave_n;
+    __syncthreads();
+    unsigned pos = offset + before;
+#pragma unroll
+    for (unsigned w = 0; w < kBlock / 64; ++w) {
+      if (w < wave) pos += wave_cnt[w];
+      offset += wave_cnt[w];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (hit[j]) {
+        if (pos < cap) {
+          oidx[pos] = (int32_t)(base + 4 * (int64_t)(threadIdx.x + kBlock * r) + j);
+          osnr[pos] = v[j];
+        }
+        ++pos;
       }
-    }
-    offset += n_round;
-    __syncthreads();
   }
 }
 
@@ -435,38 +632,21 @@ extern "C" int psx_deredden_median(const float* A, uint64_t nb, double bin_width
   float* m5 = work;
   float* m25 = m5 + c5 + 1;
   float* m125 = m25 + c25 + 1;
-  int rc;
-  if ((rc = psx_median_scrunch5(A, nb, m5, s))) return rc;
-  if ((rc = psx_median_scrunch5(m5, c5, m25, s))) return rc;
-  if ((rc = psx_median_scrunch5(m25, c25, m125, s))) return rc;
+  const hipStream_t hs = as_stream(s);
+  k_scrunch125<<<(unsigned)((c5 + 25 * kM125 - 1) / (25 * kM125)), kBlock, 0, hs>>>(A, m5, m25, m125, c5, c25, c125);
+  PSX_CHECK_LAUNCH("k_scrunch125");
   const int64_t pos5 = (int64_t)(int)((double)b5 / bin_width);
   const int64_t pos25 = (int64_t)(int)((double)b25 / bin_width);
   auto clampz = [&](int64_t v) -> uint64_t { return v < 0 ? 0 : (v > (int64_t)nb ? nb : (uint64_t)v); };
-  const uint64_t z0 = 0, z1 = clampz(pos5), z2 = clampz(pos25);
-  const hipStream_t hs = as_stream(s);
-  // zone [0, pos5) <- m5
-  if (z1 > z0) {
-    k_stretch_zone<<<psx::grid_for(z1 - z0, kBlock), kBlock, 0, hs>>>(m5, c5, median, z0, z1, psx::stretch_step(c5, nb));
-    PSX_CHECK_LAUNCH("k_stretch_zone");
-  }
-  // zone [pos5, pos25) <- m25 (the reference copies pos25 elements from pos5;
-  // everything from pos25 on is rewritten by the third zone)
-  const uint64_t z1e = clampz(pos5 + pos25);
-  const uint64_t hi25 = z2 > z1 ? z2 : z1;
-  if (z1e > z1) {
-    const uint64_t hi = z1e < hi25 ? z1e : hi25;
-    if (hi > z1) {
-      k_stretch_zone<<<psx::grid_for(hi - z1, kBlock), kBlock, 0, hs>>>(m25, c25, median, z1, hi,
-                                                                        psx::stretch_step(c25, nb));
-      PSX_CHECK_LAUNCH("k_stretch_zone");
-    }
-  }
-  // zone [pos25, nb) <- m125
-  if (nb > z2) {
-    k_stretch_zone<<<psx::grid_for(nb - z2, kBlock), kBlock, 0, hs>>>(m125, c125, median, z2, nb,
-                                                                      psx::stretch_step(c125, nb));
-    PSX_CHECK_LAUNCH("k_stretch_zone");
-  }
+  // zone [0, pos5) <- m5, zone [pos5, pos25) <- m25 (the reference copies
+  // pos25 elements from pos5; everything from pos25 on is rewritten by the
+  // third zone), zone [pos25, nb) <- m125
+  const uint64_t z1 = clampz(pos5), z2 = clampz(pos25);
+  const uint64_t hi = std::min(clampz(pos5 + pos25), std::max(z1, z2));
+  k_stretch_zones<<<psx::grid_for(nb, kBlock), kBlock, 0, hs>>>(
+      Stretch{m5, c5, psx::stretch_step(c5, nb)}, Stretch{m25, c25, psx::stretch_step(c25, nb)},
+      Stretch{m125, c125, psx::stretch_step(c125, nb)}, z1, hi, z2, median, nb);
+  PSX_CHECK_LAUNCH("k_stretch_zones");
   return psx::ok();
 }
 
@@ -557,21 +737,34 @@ extern "C" int psx_normalise(float* p, float mean, float sigma, uint64_t n, psx_
   return psx::ok();
 }
 
-// GPU_remove_baseline (src/kernels.cu:463-479).
+// GPU_remove_baseline (src/kernels.cu:463-479): two iterations per look at
+// the loop's state (series need one or two).
 extern "C" int psx_remove_baseline(float* x, uint64_t n, void* work, psx_stream s) {
   PSX_REQUIRE(x && work && n > 0, "psx_remove_baseline: bad arguments");
-  int count = 0;
-  float mean;
+  const hipStream_t hs = as_stream(s);
+  double2* partial = (double2*)work;
+  BaselineState* st = (BaselineState*)(partial + kReduceBlocks);  // two states
+  static_assert(2 * sizeof(BaselineState) <= sizeof(double2), "states in the total's place");
+  const unsigned g = psx::grid_for(n, kBlock, kReduceBlocks);
+  bool first = true;
+  BaselineState h;
   do {
-    double s1, s2;
-    int rc = sum_sq(x, 0, n, work, s, &s1, &s2);
-    if (rc) return rc;
-    mean = (float)s1 / (float)(int64_t)n;
-    k_subtract<<<psx::grid_for(n, kBlock), kBlock, 0, as_stream(s)>>>(x, n, mean);
-    PSX_CHECK_LAUNCH("k_subtract");
-    if (count++ > 100) break;
-  } while (fabsf(mean) > 5e-7 * (double)n);
-  PSX_CHECK_HIP(hipStreamSynchronize(as_stream(s)));
+    for (int i = 0; i < 2; ++i) {
+      if (first) {
+        k_base_sum<true><<<g, kBlock, 0, hs>>>(x, n, partial, nullptr);
+        PSX_CHECK_LAUNCH("k_base_sum");
+        k_base_sub<true><<<g, kBlock, 0, hs>>>(x, n, partial, g, nullptr, st);
+      } else {
+        k_base_sum<false><<<g, kBlock, 0, hs>>>(x, n, partial, st + (i ^ 1));
+        PSX_CHECK_LAUNCH("k_base_sum");
+        k_base_sub<false><<<g, kBlock, 0, hs>>>(x, n, partial, g, st + (i ^ 1), st + i);
+      }
+      PSX_CHECK_LAUNCH("k_base_sub");
+      first = false;
+    }
+    PSX_CHECK_HIP(hipMemcpyAsync(&h, st + 1, sizeof(h), hipMemcpyDeviceToHost, hs));
+    PSX_CHECK_HIP(hipStreamSynchronize(hs));
+  } while (!h.done);
   return psx::ok();
 }
 
@@ -609,14 +802,13 @@ extern "C" int psx_harmonic_sum(const float* P, float* const* folds, uint32_t nf
   }
   if (!nb) return psx::ok();
   psx::TraceRange range("Harmonic summing");
-  const unsigned g = psx::grid_for(nb, kBlock);
   const hipStream_t hs = as_stream(s);
   switch (nfolds) {
-    case 1: k_harmonic<1><<<g, kBlock, 0, hs>>>(P, fp, nb); break;
-    case 2: k_harmonic<2><<<g, kBlock, 0, hs>>>(P, fp, nb); break;
-    case 3: k_harmonic<3><<<g, kBlock, 0, hs>>>(P, fp, nb); break;
-    case 4: k_harmonic<4><<<g, kBlock, 0, hs>>>(P, fp, nb); break;
-    default: k_harmonic<5><<<g, kBlock, 0, hs>>>(P, fp, nb); break;
+    case 1: launch_harmonic<1>(P, fp, nb, hs); break;
+    case 2: launch_harmonic<2>(P, fp, nb, hs); break;
+    case 3: launch_harmonic<3>(P, fp, nb, hs); break;
+    case 4: launch_harmonic<4>(P, fp, nb, hs); break;
+    default: launch_harmonic<5>(P, fp, nb, hs); break;
   }
   PSX_CHECK_LAUNCH("k_harmonic");
   return psx::ok();

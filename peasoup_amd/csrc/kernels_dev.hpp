@@ -9,6 +9,8 @@
 
 #include <cstdint>
 
+#include "common.hpp"
+
 namespace psx {
 
 // device_resampleII (src/kernels.cu:361): (a*tsamp) is a float product,
@@ -191,6 +193,45 @@ __device__ inline void harmonic_sums32(const float* __restrict__ P, uint32_t i, 
   }
 }
 
+// The same sums for D bins per lane: lane l of a wave holds the bins i0 + 64d,
+// i0 = base + l.  Fold k's harmonic j of bin i is bin (j*i + 2^(k-1)) >> k, and
+// with i = i0 + 64d that is ((j*i0 + 2^(k-1)) >> k) + d*64j/2^k exactly (2^k
+// divides 64), so each harmonic costs one index per lane and D loads at
+// constant instruction offsets from it: the gathers stay coalesced across
+// lanes and the index arithmetic drops out of the loop.  val takes the same
+// addends in the same order as harmonic_sums32 (bins below 2^27).
+//
+// Harmonics at 1/16 of the bin or less (step <= 4) touch only D*step + 1
+// consecutive bins per wave, fewer than 64: the wave loads them once (one
+// load per lane) and each d takes its value from the owning lane with
+// ds_bpermute, instead of D loads of a few distinct floats each (2% faster
+// batched harmonic pass).  The values are the same bins, so the sums are unchanged.
+template <int K, int J, int D>
+__device__ inline void add_harmonic(const PSX_GLOBAL float* p, uint32_t i0, float (&val)[D]) {
+  constexpr uint32_t step = (64u * J) >> K;
+  constexpr uint32_t c = 1u << (K - 1);
+  if constexpr (step <= 4 && D * step + 1 < 64) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t s0 = (J * (i0 - lane) + c) >> K;  // the wave's first bin of this harmonic
+    const uint32_t r = ((J * i0 + c) >> K) - s0;     // this lane's offset, <= step
+    const float chunk = p[s0 + lane];
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const int addr = (int)((r + (uint32_t)d * step) << 2);
+      val[d] += __int_as_float(__builtin_amdgcn_ds_bpermute(addr, __float_as_int(chunk)));
+    }
+  } else {
+    const PSX_GLOBAL float* q = p + ((J * i0 + c) >> K);
+#pragma unroll
+    for (int d = 0; d < D; ++d) val[d] += q[d * step];
+  }
+}
+// odd harmonics J, J+2, ... below JEND of fold K, in increasing order
+template <int K, int J, int JEND, int D>
+__device__ inline void add_harmonics(const PSX_GLOBAL float* p, uint32_t i0, float (&val)[D]) {
+  add_harmonic<K, J, D>(p, i0, val);
+  if constexpr (J + 2 < JEND) add_harmonics<K, J + 2, JEND, D>(p, i0, val);
+}
 // Number of set bits of mask in the lanes below the calling lane (wave64).
 __device__ inline unsigned mbcnt64(uint64_t mask) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
