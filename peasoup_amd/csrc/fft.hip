@@ -995,9 +995,15 @@ int exec_fused_pass(psx_fft_plan* p, int q, const TrialDesc* d_descs, uint32_t n
   if (q == 0 && L.gy != 1) return psx::fail(PSX_ERR_UNSUPPORTED, "exec_fused_pass: first pass with sub-transforms");
   unsigned gx = L.gx;
   if (k->two_tiles && gx > 1) {
-    a.tiles = kTilesPerGroup;
+    // several tiles per workgroup only while one round of workgroups still
+    // fills every CU: 8 always left 48 workgroups to a 24-trial batch of 2^17
+    // samples (row pass of 16 trials of 2^20 2.67 us per trial, now 1.78; of 4
+    // trials of 2^22 16.4, now 7.0; 64 trials unchanged)
+    const uint64_t slots = 256ull * std::min(163840 / k->lds, 2048 / k->threads);
+    const uint64_t per = (uint64_t)gx * L.gy * ntrials / slots;
+    a.tiles = (int32_t)std::min<uint64_t>(kTilesPerGroup, std::max<uint64_t>(1, per));
     a.ntiles = gx;
-    gx = (gx + kTilesPerGroup - 1) / kTilesPerGroup;
+    gx = (gx + a.tiles - 1) / a.tiles;
   }
   hipLaunchKernelGGL(k->fn, dim3(gx, L.gy, ntrials), dim3(k->threads), k->lds, hs, a);
   PSX_CHECK_LAUNCH("k_fft_pass(fused)");
