@@ -279,10 +279,11 @@ enum { PSX_SPECTRUM_AUTO = 0, PSX_SPECTRUM_NATURAL = 1, PSX_SPECTRUM_ROWS = 2 };
 
 /* Harmonic-sum pass of the batched path (harmonic_sum_kernel + PeakFinder,
  * src/kernels.cu:34-100,391-423).  BOUND: a pooled bfloat16 copy of
- * each spectrum (every entry rounded up from the larger of two bins) is
- * summed in the reference's addend order; since every addend and every
- * rounding step only grows, those sums bound the exact fold sums from
- * above, and only bins whose bound crosses the threshold are summed exactly.
+ * each spectrum (every entry rounded up from the largest of three bins) is
+ * summed in the reference's addend order for two bins at a time; since every
+ * addend and every rounding step only grows, those sums bound the exact fold
+ * sums from above, and only bins whose bound crosses the threshold are summed
+ * exactly.
  * EXACT: every addend of every bin gathered from the spectrum.  Both give
  * identical candidates; BOUND moves about a third of the memory traffic. */
 enum { PSX_HARMONIC_BOUND = 0, PSX_HARMONIC_EXACT = 1 };
@@ -318,13 +319,13 @@ int psx_batch_profile(const psx_search_args* args, const psx_batch_opts* opts, c
  * in the reference): runs the prologue of d_series and the FFT and spectrum
  * stages of one batch (min(naccs, batch) trials), has the exact spectra P
  * written from the same FFT output, and checks on the host every bound
- * entry against max(P[2u], P[2u+1]) and the fundamental's candidates against
- * the bins above threshold.  result[0] = entries checked, [1] = entries below
- * their pair's maximum (invalid bounds: 0 when correct), [2] = fundamental
- * bins above threshold on the host, [3] = candidates the device appended
- * (equal to [2] when correct), [4] = bins of the harmonic window whose bound
- * sums cross at some fold (the bins summed exactly), [5] = bins of the
- * window, [6] = valid entries above the tight bound (the pair maximum
+ * entry against max(P[2u-1], P[2u], P[2u+1]) and the fundamental's candidates
+ * against the bins above threshold.  result[0] = entries checked, [1] =
+ * entries below their bins' maximum (invalid bounds: 0 when correct), [2] =
+ * fundamental bins above threshold on the host, [3] = candidates the device
+ * appended (equal to [2] when correct), [4] = bins of the harmonic window
+ * whose bound sums cross at some fold (the bins summed exactly), [5] = bins of
+ * the window, [6] = valid entries above the tight bound (the bins' maximum
  * rounded up to bfloat16; the row-layout pass bounds each value from
  * approximate arithmetic and may land one step higher).  result holds 7
  * values.  For tests and for validating a new FFT decomposition. */

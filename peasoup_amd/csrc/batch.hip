@@ -4,9 +4,9 @@
 //   k_fft_pass (resample fused into the first pass) ... FFT passes -> Z
 //   k_spec_post   untangle + interbin + normalise          Z -> P
 //   k_pool_peaks  fundamental threshold + bound spectrum   P -> Q, candidates
-//   k_harm_bound  2..2^F harmonic sums over Q (an upper bound of every
-//                 fold sum); exact sums of P where a bound
-//                 crosses the threshold                    Q, P -> candidates
+//   k_harm_bound  2..2^F harmonic sums over Q (upper bounds of the fold
+//                 sums, two bins at a time); exact sums of P
+//                 where a bound crosses the threshold      Q, P -> candidates
 // (k_harm_peaks, the exact sums of every bin, is the alternative harmonic
 // pass: same candidates, more memory traffic.)
 // The per-trial arithmetic is the plain path's, operation for operation
@@ -104,8 +104,36 @@ __device__ inline void lds_bf16x8(const uint16_t* e, float (&t)[8]) {
         "i"(12 * STRIDE), "i"(14 * STRIDE));
 }
 
+// The same for two runs of entries under one wait.
+template <int S1, int S2>
+__device__ inline void lds_bf16x16(const uint16_t* e, const uint16_t* e2, float (&t)[8], float (&u)[8]) {
+  const uint32_t a = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint16_t*)e;
+  const uint32_t b = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint16_t*)e2;
+  asm volatile(
+      "ds_read_u16_d16_hi %0, %16\n\t"
+      "ds_read_u16_d16_hi %1, %16 offset:1*%18\n\t"
+      "ds_read_u16_d16_hi %2, %16 offset:2*%18\n\t"
+      "ds_read_u16_d16_hi %3, %16 offset:3*%18\n\t"
+      "ds_read_u16_d16_hi %4, %16 offset:4*%18\n\t"
+      "ds_read_u16_d16_hi %5, %16 offset:5*%18\n\t"
+      "ds_read_u16_d16_hi %6, %16 offset:6*%18\n\t"
+      "ds_read_u16_d16_hi %7, %16 offset:7*%18\n\t"
+      "ds_read_u16_d16_hi %8, %17\n\t"
+      "ds_read_u16_d16_hi %9, %17 offset:1*%19\n\t"
+      "ds_read_u16_d16_hi %10, %17 offset:2*%19\n\t"
+      "ds_read_u16_d16_hi %11, %17 offset:3*%19\n\t"
+      "ds_read_u16_d16_hi %12, %17 offset:4*%19\n\t"
+      "ds_read_u16_d16_hi %13, %17 offset:5*%19\n\t"
+      "ds_read_u16_d16_hi %14, %17 offset:6*%19\n\t"
+      "ds_read_u16_d16_hi %15, %17 offset:7*%19\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "+v"(t[0]), "+v"(t[1]), "+v"(t[2]), "+v"(t[3]), "+v"(t[4]), "+v"(t[5]), "+v"(t[6]), "+v"(t[7]),
+        "+v"(u[0]), "+v"(u[1]), "+v"(u[2]), "+v"(u[3]), "+v"(u[4]), "+v"(u[5]), "+v"(u[6]), "+v"(u[7])
+      : "v"(a), "v"(b), "i"(2 * S1), "i"(2 * S2));
+}
+
 // Outputs of the spectrum pass for the bound-filtered harmonic pass: the
-// bound spectrum (one bfloat16 upper bound per bin pair 2u, 2u+1) and
+// bound spectrum (one bfloat16 upper bound of the bins 2u-1, 2u, 2u+1) and
 // the fundamental's above-threshold bins (device_find_peaks over
 // PeakFinder's nh = 0 window, src/kernels.cu:391-423, peakfinder.hpp:78-83).
 struct BoundOut {
@@ -238,9 +266,9 @@ __device__ inline float2 x_rows(const float2* y, uint32_t R, uint32_t L, uint32_
   return xk;
 }
 // t < L: row 0; t < 2L: row R/2; t == 2L: bin M.  Returns the bin and its
-// value; with bo, also the bound of the bin pair (k, k+1), whose second bin
-// (row 1 or R/2 + 1, a tile's) is recomputed here through the same untangle
-// and interbin arithmetic, so it equals the tile's value bit for bit.
+// value; with BOUND, also the bound of the bins k-1, k, k+1 (k is even), whose
+// outer ones (other rows' bins) are recomputed here through the same untangle
+// and interbin arithmetic.
 template <bool BOUND>
 __device__ inline float spec_edge_bin(const float2* y, float* p, uint32_t R, uint32_t L, uint32_t t,
                                       const RootTable& rt, float mean_n, float std_n, uint16_t* q, uint32_t& k) {
@@ -258,8 +286,13 @@ __device__ inline float spec_edge_bin(const float2* y, float* p, uint32_t R, uin
   const float v = normalised(x, prev, mean_n, std_n);
   if constexpr (!BOUND) p[k] = v;
   if constexpr (BOUND) {
-    float m = v;  // bin M has no partner (n/2 + 1 bins)
-    if (k < M) m = fmaxf(v, normalised(x_rows(y, R, L, k + 1, rt), x, mean_n, std_n));
+    float m = v;
+    if (k > 0) {
+      const float2 prev2 = k > 1 ? x_rows(y, R, L, k - 2, rt) : make_float2(0.f, 0.f);
+      m = fmaxf(m, normalised(prev, prev2, mean_n, std_n));
+    }
+    // bin M is the last
+    if (k < M) m = fmaxf(m, normalised(x_rows(y, R, L, k + 1, rt), x, mean_n, std_n));
     q[k / 2] = bf16_up(m);
   }
   return v;
@@ -376,21 +409,26 @@ __global__ void __launch_bounds__(kB) k_spec_rows(const float2* __restrict__ Y, 
   }
   edge_lo[wv][lane] = xlo_prev;
   xhi_last = xhi_prev;
-  float2 below = make_float2(0.f, 0.f), above = make_float2(0.f, 0.f), next_lo;
-  if (wv == 0) pair_row(ra - 1, below, next_lo);
-  if (wv == kB / 64 - 1) pair_row(ra + kRowTile, next_lo, above);
+  float2 below = make_float2(0.f, 0.f), above = make_float2(0.f, 0.f), above2 = above, next_lo, unused;
+  if (wv == 0) pair_row(ra - 1, below, unused);
+  if (wv == kB / 64 - 1) {
+    pair_row(ra + kRowTile, next_lo, above);
+    if constexpr (BOUND) pair_row(ra + kRowTile + 1, unused, above2);
+  }
   __syncthreads();
   if (wv > 0) below = edge_lo[wv - 1][lane];
   if (wv < kB / 64 - 1) above = edge_hi[wv + 1][lane];
   lo_t[lane][slot(r0)] = tile_value(xlo_first, below);
   up_t[lane][slot(r0 + kWaveRows - 1)] = tile_value(xhi_last, above);
   if constexpr (BOUND) {
-    // P of the next tile's first row (ra + 64), the partner of this tile's
-    // last row in a bound pair: its X was loaded for the upper halo, and the
-    // interbin neighbour is this tile's last row.  Slot kRowTile is free in
-    // every tile but the last, which has no such pair.
-    if (wv == kB / 64 - 1 && ra + kRowTile < half_rows)
+    // The next tile's first rows, lower (ra + 64) and upper (R - ra - 64),
+    // which the bounds of this tile's last lower and upper pairs include:
+    // their X were loaded for the halo.  Slot kRowTile is free in every tile
+    // but the last, which has no such pairs.
+    if (wv == kB / 64 - 1 && ra + kRowTile < half_rows) {
       lo_t[lane][kRowTile] = tile_value(next_lo, xlo_prev);
+      up_t[lane][kRowTile] = tile_value(above, above2);
+    }
   }
   __syncthreads();
   const uint32_t rr = threadIdx.x & 63u;
@@ -404,18 +442,17 @@ __global__ void __launch_bounds__(kB) k_spec_rows(const float2* __restrict__ Y, 
       }
     }
   } else {
-    // Bound pairs (2u, 2u+1): rows 0/1 and R/2 / R/2+1 of every column are the
-    // edge workgroups'; a tile's column holds 32 lower pairs, rows
-    // (ra+2i+1, ra+2i+2), i < 32 (slot kRowTile for the last one's second
-    // row), and 32 upper pairs, rows R-r for r = ra+63-2i and ra+62-2i.
-    // Lane i < 32 bounds lower pair i, lane 32+i upper pair i: one 16-bit
-    // store covers both runs of 32 entries.  Every value written is also
-    // tested as a fundamental.
+    // Bounds of the bins (2u-1, 2u, 2u+1): those of the even rows 0 and R/2 of
+    // every column are the edge workgroups'; a tile's column holds 32 lower
+    // ones, around rows ra+2i+1, i < 32 (slot kRowTile for the last one's
+    // third row), and 32 upper ones, around rows R-r, r = ra+63-2i (slot
+    // kRowTile for the first one's first row).  Lane i < 32 bounds lower
+    // triple i, lane 32+i upper triple i: one 16-bit store covers both runs of
+    // 32 entries.  Every value written is also tested as a fundamental.
     const bool rv = r < half_rows;
     const bool lower = rr < 32;
     const uint32_t i = rr & 31u;
-    const uint32_t s0 = lower ? 2 * i + 1 : 63 - 2 * i;  // slot of the pair's even row
-    const uint32_t s1 = lower ? s0 + 1 : s0 - 1;         // and of its odd row
+    const uint32_t s0 = lower ? 2 * i + 1 : 63 - 2 * i;  // slot of the even row; its neighbours' are beside it
     const uint32_t rpair = ra + s0;                      // lower-half row of the even-row slot
     const bool pv = rpair < half_rows;
     bool any = false;
@@ -424,7 +461,8 @@ __global__ void __launch_bounds__(kB) k_spec_rows(const float2* __restrict__ Y, 
       const float vl = lo_t[j][rr], vu = up_t[j][rr];
       if (rv) any |= fmaxf(vl, vu) > bo.thr;
       if (pv) {
-        const float m = lower ? fmaxf(lo_t[j][s0], lo_t[j][s1]) : fmaxf(up_t[j][s0], up_t[j][s1]);
+        const float* t = lower ? lo_t[j] : up_t[j];
+        const float m = fmaxf(fmaxf(t[s0 - 1], t[s0]), t[s0 + 1]);
         const uint32_t k2 = lower ? rpair + R * (ea + j) : (R - rpair) + R * (L - 1 - (ea + j));
         q[k2 / 2] = bf16_up(m);
       }
@@ -569,37 +607,40 @@ __global__ void __launch_bounds__(kB) k_harm_peaks(const float* __restrict__ P, 
 // holds a fraction of one 16 MB spectrum, and the miss path moves about
 // 7.5 TB/s whether the MALL or HBM serves it.  Candidates are rare, so this
 // form first proves most bins empty from a smaller array:
-//   Q[u] = max(P[2u], P[2u+1]) rounded up to bfloat16,
-// one 16-bit entry per two bins (a quarter of the spectrum's bytes).  Every
-// addend P[x] of a fold sum is at most Q[x/2], and float addition,
-// fold_scale and the comparison are monotone (round to nearest never
-// reverses an order), so the running sum of the Q entries taken in the
-// reference's addend order is at least the exact running sum at every fold:
-// where the bound of fold k stays at or below the threshold, so does fold
-// k's exact value.  Only the bins whose bound crosses (about 1e-6 of
-// noise bins, and every real detection) are summed exactly from P with
-// harmonic_sums32, thresholded and appended, so the candidates are the
-// gather form's bit for bit.  bfloat16 (8 significant bits) loosens the
-// bound no more than half precision does at these values (the same rate of
-// crossing noise bins in a float64 simulation), and rounds up with two
-// integer operations where half precision needs a conversion, a check and
-// a step.
+//   Q[u] = max(P[2u-1], P[2u], P[2u+1]) rounded up to bfloat16,
+// one 16-bit entry per two bins (a quarter of the spectrum's bytes), and sums
+// it for two bins at a time.  Harmonic j/2^k of the bins 2g and 2g+1 takes
+// the source bins s0 <= s1 <= s0 + 1, s1 = (j*(2g+1) + 2^(k-1)) >> k: both are
+// covered by Q[s1/2].  Float addition, fold_scale and the comparison are
+// monotone (round to nearest never reverses an order), so the running sum of
+// those entries in the reference's addend order is at least the exact running
+// sum of either bin at every fold: where the bound of fold k stays at or
+// below the threshold, so do fold k's exact values.  Only the pairs of bins
+// whose bound crosses (3e-5 of noise, and every real detection) are
+// summed exactly from P with harmonic_sums32's addends in its order,
+// thresholded and appended, so the candidates are the gather form's bit for
+// bit.  bfloat16 (8 significant bits) loosens the bound no more than half
+// precision does at these values (the same rate of crossing noise bins in a
+// float64 simulation), and rounds up with two integer operations where half
+// precision needs a conversion, a check and a step.
 //
 // fold_scale<K>(v) > thr is tested as v > T[K], T[K] the largest float
 // whose fold_scale is at most thr (found on the host by bisection over the
 // float order; fold_scale is monotone), which keeps double arithmetic out
 // of the loop.
 //
-// A wave covers kBoundWaveBins consecutive bins, lane l holding bins
-// base + l + 64d (d < 8), as in the gather form.  Harmonic j/2^k of those
-// 512 bins takes its addends from at most 512j/2^k + 1 consecutive source
-// bins, one run of 256j/2^k + 1 entries of Q; the wave copies every run (and
-// the fundamental's) into its own LDS area with global_load_lds_dwordx4
-// (one instruction per run, 16 bytes per lane, no registers), waits once,
-// and then reads each addend from LDS at a constant offset per d.  The
-// wave's LDS area is private: no barriers.  Measured at 2^23 with 64 trials
-// per launch: 0.36 ms against 0.80 ms for the gather form, the same
-// candidates; writing the bounds costs the spectrum pass about 0.1 ms.
+// A wave covers kBoundWavePairs pairs of bins, lane l holding the pairs
+// base + l + 64d (d < 8).  Harmonic j/2^k takes its addends from one run of
+// at most kBoundWavePairs*j/2^k + 2 entries of Q; the wave copies every run (and the
+// fundamental's) into its own LDS area with global_load_lds_dwordx4 (one
+// instruction per run, 16 bytes per lane, no registers), waits once, and then
+// reads each addend from LDS at a constant offset per d, two harmonics per
+// wait.  A workgroup is one wave, so its 9 KB of LDS free up by themselves (16
+// waves per CU).  Per 64 trials of 2^23: 0.80 ms the gather form, 0.34-0.36 ms
+// with max(P[2u], P[2u+1]) summed for every bin, 0.26 ms for two bins at a
+// time in workgroups of four waves, 0.24 ms in workgroups of one with two
+// harmonics per wait.  Bound by its some 330 vector instructions per wave and
+// the LDS and L2 latencies that four waves per SIMD leave uncovered.
 
 // Harmonic h (0-based, in the reference's addend order, fold 2 taking 3/4
 // before 1/4) is j/2^k with k = hK(h), j = hJ(h); fold k ends at h = 2^k - 2.
@@ -608,20 +649,19 @@ __host__ __device__ constexpr int hJ(int h) {
   return h == 0 ? 1 : h == 1 ? 3 : h == 2 ? 1 : h < 7 ? 2 * (h - 3) + 1 : h < 15 ? 2 * (h - 7) + 1 : 2 * (h - 15) + 1;
 }
 constexpr int kBoundChunk = 8;  // entries per 16-byte chunk
-constexpr int kBoundD = kBoundWaveBins / 64;
-// chunks of harmonic h's run: its sources span at most j*W/2^k bins, W/2^k/2
-// entries, plus one entry and the chunk alignment
+constexpr int kBoundD = kBoundWavePairs / 64;
+// chunks of harmonic h's run: W*j/2^k + 2 entries and the chunk alignment
 __host__ __device__ constexpr int run_chunks(int h) {
-  return ((hJ(h) * (int)kBoundWaveBins >> hK(h)) / (int)kBoundPool) / kBoundChunk + 2;
+  return (hJ(h) * (int)kBoundWavePairs >> hK(h)) / kBoundChunk + 2;
 }
-// LDS offset (entries) of run h; the fundamental's run (W/2 entries + the
-// alignment) comes first, at 0
+// LDS offset (entries) of run h; the fundamental's run (W entries, aligned)
+// comes first, at 0
 __host__ __device__ constexpr int run_offset(int h) {
-  int r = ((int)kBoundWaveBins / (int)kBoundPool / kBoundChunk + 1) * kBoundChunk;
+  int r = (int)kBoundWavePairs;
   for (int g = 0; g < h; ++g) r += run_chunks(g) * kBoundChunk;
   return r;
 }
-static_assert(run_chunks(30) <= 64 && (int)kBoundWaveBins / (int)kBoundPool / kBoundChunk + 1 <= 64,
+static_assert(run_chunks(30) <= 64 && (int)kBoundWavePairs / kBoundChunk <= 64 && kBoundWavePairs % kBoundChunk == 0,
               "one 64-lane instruction per run");
 
 typedef float psx_f4v __attribute__((ext_vector_type(4)));
@@ -646,6 +686,9 @@ __global__ void __launch_bounds__(kB) k_pool_peaks(const float* __restrict__ P, 
     const uint32_t g = g0 + lane;
     const uint32_t k0 = 4 * g;
     float x[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    // the bin before the wave's first (an entry includes the bin below its pair)
+    float before = -INFINITY;
+    if (lane == 0 && k0 > 0) before = p[k0 - 1];
     if (g < ngroups) {
       // k0 + 3 < pstride: rows are padded to a multiple of 64 bins
       const psx_f4v v = __builtin_nontemporal_load((const PSX_GLOBAL psx_f4v*)(p + k0));
@@ -653,7 +696,12 @@ __global__ void __launch_bounds__(kB) k_pool_peaks(const float* __restrict__ P, 
       x[1] = k0 + 1 < nb ? v.y : -INFINITY;
       x[2] = k0 + 2 < nb ? v.z : -INFINITY;
       x[3] = k0 + 3 < nb ? v.w : -INFINITY;
-      const uint32_t pair = (uint32_t)bf16_up(fmaxf(x[0], x[1])) | ((uint32_t)bf16_up(fmaxf(x[2], x[3])) << 16);
+    }
+    const float last = __shfl_up(x[3], 1);
+    if (lane > 0) before = last;
+    if (g < ngroups) {
+      const uint32_t pair = (uint32_t)bf16_up(fmaxf(fmaxf(before, x[0]), x[1])) |
+                            ((uint32_t)bf16_up(fmaxf(fmaxf(x[1], x[2]), x[3])) << 16);
       *(PSX_GLOBAL uint32_t*)(q + 2 * g) = pair;
     }
     bool any = false;
@@ -694,37 +742,53 @@ __device__ inline uint32_t stage_run(const PSX_GLOBAL uint16_t* q, uint32_t s0, 
   return a0;
 }
 
+// Entry of Q that covers harmonic J/2^K of the pair of bins g.
+template <int K, int J>
+__device__ inline uint32_t pair_entry(uint32_t g) {
+  return ((J * (2 * g + 1) + (1u << (K - 1))) >> K) >> 1;
+}
+
 template <int NH, int H>
 struct BoundRuns {
-  __device__ static void stage(const PSX_GLOBAL uint16_t* q, uint32_t base, uint16_t* my, uint32_t (&a0)[NH + 1],
+  __device__ static void stage(const PSX_GLOBAL uint16_t* q, uint32_t base, uint16_t* my, uint32_t (&a0)[NH],
                                unsigned lane) {
     if constexpr (H < NH) {
       constexpr int K = hK(H), J = hJ(H);
-      constexpr uint32_t c = 1u << (K - 1);
-      a0[H] = stage_run(q, ((J * base + c) >> K) / kBoundPool,
-                        ((J * (base + kBoundWaveBins - 1) + c) >> K) / kBoundPool, my + run_offset(H), lane);
+      a0[H] = stage_run(q, pair_entry<K, J>(base), pair_entry<K, J>(base + kBoundWavePairs - 1), my + run_offset(H),
+                        lane);
       BoundRuns<NH, H + 1>::stage(q, base, my, a0, lane);
     }
   }
-  // adds harmonic H's bound to every running sum; at a fold's last addend
-  // marks the bins whose bound crosses that fold's threshold
-  __device__ static void add(const uint16_t* my, const uint32_t (&a0)[NH + 1], uint32_t i0, const FoldThr& ft,
-                             float (&val)[kBoundD], bool (&fail)[kBoundD], float (&t)[kBoundD]) {
+  // adds the bounds of harmonics H and H + 1 (alone: harmonic 0) to every
+  // running sum; at a fold's last addend marks the pairs whose bound crosses
+  // that fold's threshold
+  __device__ static void add(const uint16_t* my, const uint32_t (&a0)[NH], uint32_t g0, const FoldThr& ft,
+                             float (&val)[kBoundD], bool (&fail)[kBoundD], float (&t)[kBoundD],
+                             float (&u)[kBoundD]) {
     if constexpr (H < NH) {
-      constexpr int K = hK(H), J = hJ(H);
-      constexpr uint32_t c = 1u << (K - 1);
-      constexpr uint32_t step = (64u * J) >> K;  // source step between a lane's bins
-      static_assert(step % kBoundPool == 0, "constant LDS offsets per d");
-      const uint16_t* b = my + run_offset(H) + (((J * i0 + c) >> K) / kBoundPool - a0[H]);
-      static_assert(kBoundD == 8, "lds_bf16x8 reads eight entries");
-      lds_bf16x8<step / kBoundPool>(b, t);
+      constexpr int H2 = H == 0 ? H : H + 1;
+      constexpr int K = hK(H), J = hJ(H), K2 = hK(H2), J2 = hJ(H2);
+      // entries between a lane's pairs: 128 bins apart, 128J/2^K source bins
+      static_assert((64 * J) % (1 << K) == 0 && (64 * J2) % (1 << K2) == 0, "constant LDS offsets per d");
+      static_assert(kBoundD == 8, "eight entries per run");
+      const uint16_t* b = my + run_offset(H) + (pair_entry<K, J>(g0) - a0[H]);
+      if constexpr (H == 0) {
+        lds_bf16x8<((64 * J) >> K)>(b, t);
+      } else {
+        const uint16_t* b2 = my + run_offset(H2) + (pair_entry<K2, J2>(g0) - a0[H2]);
+        lds_bf16x16<((64 * J) >> K), ((64 * J2) >> K2)>(b, b2, t, u);
+      }
 #pragma unroll
       for (int d = 0; d < kBoundD; ++d) val[d] += t[d];
-      if constexpr (((H + 2) & (H + 1)) == 0) {  // H = 2^K - 2: fold K complete
+      if constexpr (H > 0) {
 #pragma unroll
-        for (int d = 0; d < kBoundD; ++d) fail[d] |= val[d] > ft.t[K];
+        for (int d = 0; d < kBoundD; ++d) val[d] += u[d];
       }
-      BoundRuns<NH, H + 1>::add(my, a0, i0, ft, val, fail, t);
+      if constexpr (((H2 + 2) & (H2 + 1)) == 0) {  // H2 = 2^K - 2: fold K complete
+#pragma unroll
+        for (int d = 0; d < kBoundD; ++d) fail[d] |= val[d] > ft.t[K2];
+      }
+      BoundRuns<NH, H2 + 1>::add(my, a0, g0, ft, val, fail, t, u);
     }
   }
 };
@@ -740,6 +804,10 @@ struct ExactSrc {
   uint32_t rshift;     // log2(R) for a power of two, else 32
   RootTable rt;
 };
+// First pair of the first wave: the window's, at a whole chunk of entries.
+__host__ __device__ inline uint32_t bound_first_pair(int64_t lo) {
+  return ((uint32_t)lo / 2) & ~(uint32_t)(kBoundChunk - 1);
+}
 // harmonic_sums32's sums (the same addends in the same order) with the
 // spectrum value of bin x given by f(x), one addend per iteration of a loop
 // the compiler keeps rolled: this path runs for the rare bins whose bound
@@ -760,21 +828,46 @@ __device__ inline void harmonic_sums_rolled(F f, uint32_t i, float (&s)[5]) {
   }
 }
 
-// Register budget: eight waves per SIMD (the LDS runs allow eight
-// four-wave workgroups per CU) up to four folds; the rare exact path's
-// scalar registers would otherwise take one of them.
-constexpr int bound_waves(int nf) { return nf <= 4 ? 8 : 3; }
+// The exact folds of the two bins of pair g (the same for all lanes): lane
+// h < 2^NF of each half wave takes addend h of bin 2g + half, all of them at
+// once, and then sums them in harmonic_sums32's order; lane k < NF of a half
+// has fold k + 1.  A crossing pair costs one round of the addends' loads this
+// way, where one lane walking through its addends pays their latency 2^NF
+// times.
+template <int NF, class F>
+__device__ inline void pair_folds(F f, uint32_t g, uint32_t hi, uint32_t& i, float& s) {
+  const uint32_t lane = threadIdx.x & 63u, h = lane & 31u;
+  i = 2 * g + (lane >> 5);
+  float v = 0.f;
+  if (h < (1u << NF) && i < hi) {
+    const int K = hK((int)h - 1), J = hJ((int)h - 1);
+    v = f(h == 0 ? i : ((uint32_t)J * i + (1u << (K - 1))) >> K);
+  }
+  const int first = (int)(lane & 32u);
+  float val = __shfl(v, first);
+  s = 0.f;
+#pragma unroll
+  for (int a = 0; a < (1 << NF) - 1; ++a) {
+    val += __shfl(v, first + 1 + a);
+    if (a == 0 && h == 0) s = psx::fold_scale<1>(val);
+    if (a == 2 && h == 1) s = psx::fold_scale<2>(val);
+    if (a == 6 && h == 2) s = psx::fold_scale<3>(val);
+    if (a == 14 && h == 3) s = psx::fold_scale<4>(val);
+    if (a == 30 && h == 4) s = psx::fold_scale<5>(val);
+  }
+}
+// Pairs of one lane row (d) up to which the wave takes them one after the
+// other; where more cross (thresholds inside the noise) each lane sums its own.
+constexpr int kSerialPairs = 8;
 
 template <int NF, bool FROM_ROWS>
-__global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(bound_waves(NF)))) k_harm_bound(const float* __restrict__ P, int64_t pstride,
-                                                   const uint16_t* __restrict__ Q, int64_t qstride, Windows w,
-                                                   FoldThr ft, const TrialDesc* __restrict__ descs,
-                                                   const ExactSrc* __restrict__ srcp,
-                                                   uint32_t xcd_order, Cand16* __restrict__ out, uint32_t cap,
-                                                   uint32_t* __restrict__ count) {
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NF <= 4 ? 4 : 2)))
+k_harm_bound(const float* __restrict__ P, int64_t pstride, const uint16_t* __restrict__ Q, int64_t qstride, Windows w,
+             FoldThr ft, const TrialDesc* __restrict__ descs, const ExactSrc* __restrict__ srcp, uint32_t xcd_order,
+             Cand16* __restrict__ out, uint32_t cap, uint32_t* __restrict__ count) {
   constexpr int NH = (1 << NF) - 1;
   constexpr int WE = run_offset(NH);  // LDS entries per wave
-  __shared__ uint16_t lds[WE * (kB / 64)];
+  __shared__ __align__(16) uint16_t my[WE];
   uint32_t tr = blockIdx.y, bx = blockIdx.x;
   if (xcd_order) {
     // workgroups reach the 8 XCDs round robin: hardware block b runs on XCD
@@ -789,83 +882,90 @@ __global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(bound_w
   const float* p = P + (int64_t)tr * pstride;
   const PSX_GLOBAL uint16_t* qg = (const PSX_GLOBAL uint16_t*)(Q + (int64_t)tr * qstride);
   const unsigned lane = threadIdx.x & 63u;
-  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  uint16_t* my = lds + wave * WE;
   const uint32_t hi = (uint32_t)w.hi;
-  const uint32_t wstep = gridDim.x * (kB / 64) * kBoundWaveBins;
+  const uint32_t wstep = gridDim.x * kBoundWavePairs;
   // registers the bound entries are read into, high halves only: their low
   // halves stay zero for the whole kernel
-  float t[kBoundD];
+  float t[kBoundD], u[kBoundD];
 #pragma unroll
-  for (int d = 0; d < kBoundD; ++d) t[d] = 0.f;
-  for (uint32_t base = (uint32_t)w.lo + (bx * (kB / 64) + wave) * kBoundWaveBins; base < hi; base += wstep) {
-    const uint32_t i0 = base + lane;
+  for (int d = 0; d < kBoundD; ++d) t[d] = u[d] = 0.f;
+  for (uint32_t base = bound_first_pair(w.lo) + bx * kBoundWavePairs; 2 * base < hi; base += wstep) {
+    const uint32_t g0 = base + lane;
     // the previous tile's LDS reads are complete before the area is refilled
     __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    uint32_t a0[NH + 1];
-    a0[NH] = stage_run(qg, base / kBoundPool, (base + kBoundWaveBins - 1) / kBoundPool, my, lane);
+    uint32_t a0[NH];
+    stage_run(qg, base, base + kBoundWavePairs - 1, my, lane);
     BoundRuns<NH, 0>::stage(qg, base, my, a0, lane);
     __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
     float val[kBoundD];
     bool fail[kBoundD];
-    lds_bf16x8<64 / kBoundPool>(my + (i0 / kBoundPool - a0[NH]), t);
+    lds_bf16x8<64>(my + lane, t);
 #pragma unroll
     for (int d = 0; d < kBoundD; ++d) {
       val[d] = t[d];
       fail[d] = false;
     }
-    BoundRuns<NH, 0>::add(my, a0, i0, ft, val, fail, t);
+    BoundRuns<NH, 0>::add(my, a0, g0, ft, val, fail, t, u);
     bool any = false;
 #pragma unroll
     for (int d = 0; d < kBoundD; ++d) any |= fail[d];
     if (__ballot(any) == 0) continue;
-    // exact folds of the bins whose bound crossed (the fundamental is the
-    // pooling pass's)
+    // exact folds of the pairs whose bound crossed (the fundamental is the
+    // spectrum stage's)
     const uint32_t slot = descs[tr].slot;
+    // the spectrum's value: read from P, or recomputed from the FFT output
+    // (the source is read from memory here, not held in scalar registers by
+    // the loop)
+    auto pval = [&](uint32_t x) {
+      if constexpr (FROM_ROWS) {
+        const ExactSrc src = *srcp;
+        const float2* y = src.rows + (uint64_t)tr * (src.R * src.L);
+        const float2 xk = x_rows(y, src.R, src.L, x, src.rt, src.rshift);
+        const float2 prev = x > 0 ? x_rows(y, src.R, src.L, x - 1, src.rt, src.rshift) : make_float2(0.f, 0.f);
+        return normalised(xk, prev, descs[tr].mean_n, descs[tr].std_n);
+      } else {
+        return p[x];
+      }
+    };
+    // appends the hits (bin i, fold k + 1, value s) of the calling lanes
+    auto append = [&](bool hit, uint32_t i, uint32_t k, float s) {
+      const uint64_t mask = __ballot(hit);
+      if (mask == 0) return;
+      uint32_t b = 0;
+      if (lane == 0) b = atomicAdd(count, (uint32_t)__popcll(mask));
+      b = __shfl(b, 0);
+      if (hit) {
+        const uint32_t pos = b + psx::mbcnt64(mask);
+        if (pos < cap) out[pos] = Cand16{slot, k + 1, (int32_t)i, s};
+      }
+    };
+    auto in_window = [&](uint32_t i, int k) { return (int32_t)i >= w.start[k + 1] && (int32_t)i < w.end[k + 1]; };
 #pragma unroll
     for (int d = 0; d < kBoundD; ++d) {
-      if (__ballot(fail[d]) == 0) continue;
-      const uint32_t i = i0 + 64u * (uint32_t)d;
-      const bool valid = fail[d] && i < hi;
-      float s[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
-      if (valid) {
-        if constexpr (FROM_ROWS) {
-          // read from memory here, not held in scalar registers by the loop
-          const ExactSrc src = *srcp;
-          const uint32_t M = src.R * src.L;
-          const float2* y = src.rows + (uint64_t)tr * M;
-          const float mean_n = descs[tr].mean_n, std_n = descs[tr].std_n;
-          auto pval = [&](uint32_t x) {
-            const float2 xk = x_rows(y, src.R, src.L, x, src.rt, src.rshift);
-            const float2 prev =
-                x > 0 ? x_rows(y, src.R, src.L, x - 1, src.rt, src.rshift) : make_float2(0.f, 0.f);
-            return normalised(xk, prev, mean_n, std_n);
-          };
-          harmonic_sums_rolled<NF>(pval, i, s);
-        } else {
-          psx::harmonic_sums32<NF>(p, i, s);
-        }
-      }
-      bool hit[NF];
-      uint64_t mask[NF];
-      uint32_t total = 0;
+      uint64_t crossing = __ballot(fail[d]);
+      if (__popcll(crossing) <= kSerialPairs) {
+        while (crossing) {
+          const uint32_t g = base + 64u * (uint32_t)d + (uint32_t)__builtin_ctzll(crossing);
+          crossing &= crossing - 1;
+          uint32_t i;
+          float s;
+          pair_folds<NF>(pval, g, hi, i, s);
+          const uint32_t k = lane & 31u;
+          bool in = false;
 #pragma unroll
-      for (int k = 0; k < NF; ++k) {
-        hit[k] = valid && (int32_t)i >= w.start[k + 1] && (int32_t)i < w.end[k + 1] && s[k] > w.thr;
-        mask[k] = __ballot(hit[k]);
-        total += (uint32_t)__popcll(mask[k]);
-      }
-      if (total == 0) continue;
-      uint32_t b = 0;
-      if (lane == 0) b = atomicAdd(count, total);
-      b = __shfl(b, 0);
-#pragma unroll
-      for (int k = 0; k < NF; ++k) {
-        if (hit[k]) {
-          const uint32_t pos = b + psx::mbcnt64(mask[k]);
-          if (pos < cap) out[pos] = Cand16{slot, (uint32_t)(k + 1), (int32_t)i, s[k]};
+          for (int f = 0; f < NF; ++f) in |= k == (uint32_t)f && in_window(i, f);
+          append(in && i < hi && s > w.thr, i, k, s);
         }
-        b += (uint32_t)__popcll(mask[k]);
+      } else {
+#pragma unroll 1
+        for (uint32_t b = 0; b < 2; ++b) {
+          const uint32_t i = 2 * (g0 + 64u * (uint32_t)d) + b;
+          const bool valid = fail[d] && i < hi;
+          float s[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+          if (valid) harmonic_sums_rolled<NF>(pval, i, s);
+#pragma unroll
+          for (int k = 0; k < NF; ++k) append(valid && in_window(i, k) && s[k] > w.thr, i, (uint32_t)k, s[k]);
+        }
       }
     }
   }
@@ -973,9 +1073,9 @@ float fold_threshold_of(int k, float thr) {
 }
 
 int64_t bound_stride(int64_t pstride) {
-  // a wave's staging reads up to kBoundWaveBins - 1 bins past the window
+  // a wave's staging reads up to kBoundWavePairs - 1 entries past the window
   // end, plus a chunk of alignment: per-row slack covers both
-  return (pstride + kBoundWaveBins) / kBoundPool + 64;
+  return pstride / 2 + kBoundWavePairs + 64;
 }
 
 int launch_pool_peaks(const float* P, int64_t pstride, uint64_t nb, const Windows& w, uint16_t* Q, int64_t qstride,
@@ -1013,12 +1113,13 @@ int launch_harm_bound(const float* P, int64_t pstride, const uint16_t* Q, int64_
   const ExactSrc* src = rows ? (const ExactSrc*)d_rows_src : nullptr;
   FoldThr ft{};
   for (int k = 1; k <= 5; ++k) ft.t[k] = fold_threshold_of(k, w.thr);
-  const unsigned gx = psx::grid_for((uint64_t)(w.hi - w.lo), (uint64_t)kBoundWaveBins * (kB / 64), 2048);
+  const uint64_t pairs = ((uint64_t)w.hi + 1) / 2 - bound_first_pair(w.lo);
+  const unsigned gx = psx::grid_for(pairs, kBoundWavePairs, 1u << 16);
   const uint32_t xcd = ntr % 8 == 0 ? 1u : 0u;
   const dim3 g(gx, ntr);
   const uint16_t* q = Q;
 #define PSX_HB(NF, FR) \
-  k_harm_bound<NF, FR><<<g, kB, 0, s>>>(P, pstride, q, qstride, w, ft, d_descs, src, xcd, out, cap, count)
+  k_harm_bound<NF, FR><<<g, 64, 0, s>>>(P, pstride, q, qstride, w, ft, d_descs, src, xcd, out, cap, count)
   const bool fr = rows != nullptr;
   switch (nfolds) {
     case 1: fr ? PSX_HB(1, true) : PSX_HB(1, false); break;

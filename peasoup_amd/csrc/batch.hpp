@@ -57,12 +57,12 @@ int launch_harm_peaks(const float* P, int64_t pstride, const Windows& w, uint32_
                       const psx::fft::TrialDesc* d_descs, uint32_t ntr, Cand16* out, uint32_t cap, uint32_t* count,
                       hipStream_t s);
 // Bound-filtered harmonic pass.  Q holds, per trial row of qstride 16-bit
-// entries, bfloat16 upper bounds of bin pairs (entry u >= P[2u] and
-// P[2u+1], rounded up); launch_pool_peaks writes it from P together with
-// the fundamental's above-threshold bins, launch_harm_bound appends the
-// folds' (nh >= 1) from Q, summing P exactly only where a bound crosses.
-constexpr uint32_t kBoundPool = 2;         // bins per entry of Q
-constexpr uint32_t kBoundWaveBins = 512;   // bins per wave of k_harm_bound
+// entries, bfloat16 upper bounds of overlapping triples of bins (entry u >=
+// P[2u-1], P[2u] and P[2u+1], rounded up); launch_pool_peaks writes it from P
+// together with the fundamental's above-threshold bins, launch_harm_bound
+// appends the folds' (nh >= 1) from Q, summing P exactly only where a bound
+// crosses.
+constexpr uint32_t kBoundWavePairs = 512;  // pairs of bins per wave of k_harm_bound
 // The largest float v with fold_scale<k>(v) <= thr: fold k's running sum
 // crosses the threshold iff it exceeds this value.
 float fold_threshold_of(int k, float thr);

@@ -271,10 +271,11 @@ void Engine::audit_bounds(const TrialWork* trials, uint32_t n, BoundAudit& out) 
     const float* pr = hp.data() + (size_t)t * pstride;
     const uint16_t* qr = hq.data() + (size_t)t * qstride;
     for (uint64_t u = 0; u < nq; ++u) {
-      const float a = pr[2 * u];
-      const float m = 2 * u + 1 < nb ? std::max(a, pr[2 * u + 1]) : a;
+      float m = pr[2 * u];
+      if (u > 0) m = std::max(m, pr[2 * u - 1]);
+      if (2 * u + 1 < nb) m = std::max(m, pr[2 * u + 1]);
       out.entries++;
-      // a valid bound: its float value is at least the pair's maximum; the
+      // a valid bound: its float value is at least the triple's maximum; the
       // tight one is bf16_up_bits(m), and the fused pass (which bounds each
       // value from approximate arithmetic) may be one step above it
       const uint16_t tight = bf16_up_bits(m);
@@ -286,25 +287,26 @@ void Engine::audit_bounds(const TrialWork* trials, uint32_t n, BoundAudit& out) 
     }
     for (uint64_t k = (uint64_t)std::max(win.start[0], 0); k < (uint64_t)std::max(win.end[0], 0); ++k)
       if (pr[k] > win.thr) out.fundamentals++;
-    // the harmonic pass's bound sums, in its order and float arithmetic
+    // the harmonic pass's bound sums, in its order and float arithmetic: one
+    // for the bins 2g and 2g + 1
     float ft[6];
     for (uint32_t k = 1; k <= F; ++k) ft[k] = fold_threshold_of((int)k, win.thr);
-    auto qv = [&](uint64_t x) {
-      const uint32_t bits = (uint32_t)qr[x / 2] << 16;
+    auto qv = [&](uint64_t u) {
+      const uint32_t bits = (uint32_t)qr[u] << 16;
       float f;
       std::memcpy(&f, &bits, 4);
       return f;
     };
     for (uint64_t i = (uint64_t)win.lo; i < (uint64_t)win.hi; ++i) {
-      float val = qv(i);
+      const uint64_t odd = i | 1;
+      float val = qv(i / 2);
       bool cross = false;
-      int h = 0;
       for (uint32_t k = 1; k <= F; ++k) {
         const uint64_t c = 1ull << (k - 1);
         // fold k's odd multiples j/2^k, fold 2 taking 3/4 before 1/4
-        for (uint64_t jj = 0; jj < c; ++jj, ++h) {
+        for (uint64_t jj = 0; jj < c; ++jj) {
           const uint64_t j = (k == 2) ? (jj == 0 ? 3 : 1) : 2 * jj + 1;
-          val += qv((j * i + c) >> k);
+          val += qv(((j * odd + c) >> k) / 2);
         }
         cross |= val > ft[k];
       }

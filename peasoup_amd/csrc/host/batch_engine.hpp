@@ -54,7 +54,7 @@ struct EngineOptions {
 // Self-check of the bound spectrum one batch leaves (Engine::audit_bounds).
 struct BoundAudit {
   uint64_t entries = 0;       // bound entries checked (all trials)
-  uint64_t mismatches = 0;    // entries below the pair maximum of P (invalid bounds)
+  uint64_t mismatches = 0;    // entries below the maximum of their three bins of P (invalid bounds)
   uint64_t loose = 0;         // valid entries above the tight bound (bf16 rounding up of the maximum)
   uint64_t fundamentals = 0;  // bins above threshold in the fundamental's window (host scan of P)
   uint64_t appended = 0;      // candidates the device appended (the fundamental's, before the harmonic pass)
