@@ -2,9 +2,9 @@
 //
 // A "pass" transforms C columns of length L per workgroup.  Column c,
 // element e lives at  base + c*col_stride + e*elem_stride  in global memory;
-// the transform runs as radix-R Stockham autosort stages (R in {16,8,4,2,3})
-// whose intermediate results go through LDS.  Each thread owns P points in
-// registers; stage s assigns butterfly slot b of thread t to
+// the transform runs as radix-R Stockham autosort stages (R of 16, 8, 4, 2 and
+// 24, 12, 6, 3) whose intermediate results go through LDS.  Each thread owns P
+// points in registers; stage s assigns butterfly slot b of thread t to
 // g = b*NT + t, mapped either column-fast (c = g % C) for the global side
 // whose columns are adjacent in memory, or element-fast (j = g % (L/R)).
 // Only forward transforms are instantiated: the inverse is computed as
@@ -23,22 +23,28 @@ namespace fft {
 // ------------------------------------------------------------ radix plans
 __host__ __device__ constexpr int ilog2c(int v) { return v <= 1 ? 0 : 1 + ilog2c(v / 2); }
 __host__ __device__ constexpr bool has3(int L) { return L % 3 == 0; }
-__host__ __device__ constexpr int pow2part(int L) { return has3(L) ? L / 3 : L; }
-// Radix list: [3?] then as many 16s as fit, then the 2^r remainder.
+// Radix list of 2^m: as many 16s as fit, then the 2^r remainder.  Of 3*2^m:
+// 3*2^r first (r = m mod 3, 24 for r = 0 and m >= 3), then 8s, so that a thread
+// holds 24 points.  (With 3, 16s and the remainder it held 48: half the waves
+// per CU and a stage more.  Searches of 3*2^21 samples: a launch over rows of
+// 1,536 points in 4-row tiles 0.77 -> 0.62 ms on average, 64 trials' rows of
+// 3,072 points 1.01 -> 0.79.)
+__host__ __device__ constexpr int first_radix3(int L) {
+  const int m = ilog2c(L / 3), r = m % 3;
+  return r ? 3 << r : (m >= 3 ? 24 : 3);
+}
 __host__ __device__ constexpr int num_stages(int L) {
-  return (has3(L) ? 1 : 0) + ilog2c(pow2part(L)) / 4 + ((ilog2c(pow2part(L)) % 4) ? 1 : 0);
+  if (has3(L)) return 1 + ilog2c(L / first_radix3(L)) / 3;
+  return ilog2c(L) / 4 + ((ilog2c(L) % 4) ? 1 : 0);
 }
 __host__ __device__ constexpr int radix_at(int L, int s) {
-  return (has3(L) && s == 0) ? 3
-         : ((s - (has3(L) ? 1 : 0)) < ilog2c(pow2part(L)) / 4) ? 16
-                                                                : (1 << (ilog2c(pow2part(L)) % 4));
-}
-__host__ __device__ constexpr int max_pow2_radix(int L) {
-  return ilog2c(pow2part(L)) >= 4 ? 16 : (1 << ilog2c(pow2part(L)));
+  if (has3(L)) return s == 0 ? first_radix3(L) : 8;
+  return s < ilog2c(L) / 4 ? 16 : (1 << (ilog2c(L) % 4));
 }
 // Points per thread: a multiple of every radix of the plan.
 __host__ __device__ constexpr int points_per_thread(int L) {
-  return has3(L) ? 3 * max_pow2_radix(L) : max_pow2_radix(L);
+  if (has3(L)) return num_stages(L) == 1 ? first_radix3(L) : 24;
+  return ilog2c(L) >= 4 ? 16 : L;
 }
 __host__ __device__ constexpr int ns_before(int L, int s) { return s == 0 ? 1 : ns_before(L, s - 1) * radix_at(L, s - 1); }
 // LDS row pitch in float2: one pad slot per 16 elements plus one per row.
@@ -57,8 +63,8 @@ __host__ __device__ constexpr int lds_bytes(int L, int C, bool split) {
 // compiled for (512 / waves VGPRs), so that registers never cap the
 // workgroups per CU below what the LDS admits.  One resident workgroup per
 // CU idles the CU at every barrier and every load phase; two overlap them.
-// Plans with a radix-3 stage hold 48 points per thread (96 VGPRs of data)
-// and keep the compiler's own register allocation (target 1).
+// Plans with a factor of 3 hold 24 points per thread (48 VGPRs of data) and
+// are given at least 128 VGPRs.
 __host__ __device__ constexpr int wgs_per_cu(int L, int C, int bytes) {
   const int nt = C * L / points_per_thread(L);
   const int by_lds = 163840 / bytes;
@@ -67,7 +73,8 @@ __host__ __device__ constexpr int wgs_per_cu(int L, int C, int bytes) {
 __host__ __device__ constexpr int waves_per_simd(int L, int C, int mode) {
   const int nt = C * L / points_per_thread(L);
   const int w = (wgs_per_cu(L, C, lds_bytes(L, C, split_planes(mode))) * ((nt + 63) / 64) + 3) / 4;
-  return points_per_thread(L) > 16 ? 1 : (w > 8 ? 8 : (w < 1 ? 1 : w));
+  const int most = points_per_thread(L) > 16 ? 4 : 8;
+  return w > most ? most : (w < 1 ? 1 : w);
 }
 // Where a pass reads its stage twiddles W_L^e from.  Loading them from the
 // global table at the butterfly that uses them stalls on the load latency
@@ -77,9 +84,9 @@ __host__ __device__ constexpr int waves_per_simd(int L, int C, int mode) {
 //   TW_LDS_HALF  else its first L/2 entries, when those fit that way
 //                (W_L^(m + L/2) = -W_L^m: one sign flip per lookup);
 //   TW_PREFETCH  otherwise, when the register budget is at least 128 VGPRs
-//                and a thread holds at most 16 points, each stage's twiddles
-//                are loaded before the preceding LDS exchange (their latency
-//                hides behind it);
+//                (168 where a thread holds 24 points and 21 twiddles), each
+//                stage's twiddles are loaded before the preceding LDS exchange
+//                (their latency hides behind it);
 //   TW_GLOBAL    loads at the point of use.
 enum TwiddleSource { TW_GLOBAL = 0, TW_LDS = 1, TW_PREFETCH = 2, TW_LDS_HALF = 3 };
 // LDS twiddle tables keep entry m at slot m + m/32: a stage reads W[k*r*TS]
@@ -95,7 +102,7 @@ __host__ __device__ constexpr int twiddle_source(int L, int C, int mode) {
   const int full = tw_table_bytes(L), half = tw_table_bytes(L / 2);
   if (base + full <= 163840 && wgs_per_cu(L, C, base + full) == wgs_per_cu(L, C, base)) return TW_LDS;
   if (base + half <= 163840 && wgs_per_cu(L, C, base + half) == wgs_per_cu(L, C, base)) return TW_LDS_HALF;
-  if (points_per_thread(L) <= 16 && 512 / waves_per_simd(L, C, mode) >= 128) return TW_PREFETCH;
+  if (512 / waves_per_simd(L, C, mode) >= (points_per_thread(L) > 16 ? 168 : 128)) return TW_PREFETCH;
   return TW_GLOBAL;
 }
 // Dynamic LDS of a pass kernel: the exchange buffer plus the twiddle table.
@@ -259,13 +266,67 @@ __device__ inline void dft16(float2* v) {
   }
 }
 
+// W_24^m = exp(-2 pi i m/24), m = 0..14.
+__device__ inline float2 w24(int m) {
+  const float c1 = 0.965925826289068286749743199728897f;  // cos(pi/12)
+  const float s1 = 0.258819045102520762348898837624048f;  // sin(pi/12)
+  const float c2 = 0.866025403784438646763723170752936f;  // cos(pi/6)
+  const float h = 0.707106781186547524400844362104849f;
+  switch (m) {
+    case 0: return make_float2(1.f, 0.f);
+    case 1: return make_float2(c1, -s1);
+    case 2: return make_float2(c2, -0.5f);
+    case 3: return make_float2(h, -h);
+    case 4: return make_float2(0.5f, -c2);
+    case 5: return make_float2(s1, -c1);
+    case 6: return make_float2(0.f, -1.f);
+    case 7: return make_float2(-s1, -c1);
+    case 8: return make_float2(-0.5f, -c2);
+    case 9: return make_float2(-h, -h);
+    case 10: return make_float2(-c2, -0.5f);
+    case 11: return make_float2(-c1, -s1);
+    case 12: return make_float2(-1.f, 0.f);
+    case 13: return make_float2(-c1, s1);
+    default: return make_float2(-c2, 0.5f);  // 14
+  }
+}
+
+template <int R>
+__device__ inline void dft(float2* v);
+
+// DFT of 3M points: n = q + 3r, k = k1 + M k2, twiddle W_3M^(q*k1).
+template <int M>
+__device__ inline void dft_3m(float2* v) {
+  float2 a[3][M];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+#pragma unroll
+    for (int r = 0; r < M; ++r) a[q][r] = v[q + 3 * r];
+    dft<M>(a[q]);
+  }
+#pragma unroll
+  for (int q = 1; q < 3; ++q)
+#pragma unroll
+    for (int k1 = 1; k1 < M; ++k1) {
+      const int m = q * k1 * (8 / M);
+      a[q][k1] = m == 6 ? mul_mi(a[q][k1]) : cmul(a[q][k1], w24(m));
+    }
+#pragma unroll
+  for (int k1 = 0; k1 < M; ++k1) {
+    dft3(a[0][k1], a[1][k1], a[2][k1]);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) v[k1 + M * q] = a[q][k1];
+  }
+}
+
 template <int R>
 __device__ inline void dft(float2* v) {
   if constexpr (R == 2) dft2(v[0], v[1]);
   else if constexpr (R == 3) dft3(v[0], v[1], v[2]);
   else if constexpr (R == 4) dft4(v[0], v[1], v[2], v[3]);
   else if constexpr (R == 8) dft8(v);
-  else dft16(v);
+  else if constexpr (R == 16) dft16(v);
+  else dft_3m<R / 3>(v);
 }
 
 // ------------------------------------------------------------ pass args
@@ -312,10 +373,13 @@ struct PassArgs {
   uint32_t ntiles;
 };
 // Passes that may take two tiles per workgroup: contiguous tiles of at
-// least 4 rows whose register budget (at least 128 VGPRs) holds a second
-// tile's points while the first is transformed (narrower tiles spill).
+// least 4 rows whose register budget (at least 128 VGPRs; 256 for 24 points)
+// holds a second tile's points while the first is transformed (narrower tiles
+// spill).  Rows of 3,072 points, 64 trials of 3*2^21 samples: 1 tile 0.85 ms,
+// several 0.79; at a budget of 168 VGPRs (rows of 1,536 points, 4-row tiles)
+// they displace the prefetched twiddles, 0.68 -> 0.74.
 __host__ __device__ constexpr bool two_tiles_ok(int L, int C, int mode) {
-  return mode == 0 && C >= 4 && points_per_thread(L) <= 16 && waves_per_simd(L, C, mode) <= 4;
+  return mode == 0 && C >= 4 && waves_per_simd(L, C, mode) <= (points_per_thread(L) > 16 ? 2 : 4);
 }
 
 __device__ inline float2 tw4_lookup(const PassArgs& a, uint64_t x) {
