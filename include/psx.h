@@ -151,6 +151,17 @@ int psx_harmonic_sum(const float* P, float* const* folds, uint32_t nfolds, uint6
 uint64_t psx_find_peaks_work_bytes(uint64_t n);
 int psx_find_peaks(const float* p, int64_t start, int64_t end, float thr, int32_t* d_idx, float* d_snr,
                    uint32_t cap, uint32_t* d_count, void* work, psx_stream s);
+/* psx_find_peaks of nspec spectra (HOST arrays of device pointers and ranges)
+ * in one pair of launches.  Spectrum y's pairs go to d_idx/d_snr from
+ * y * cap, its full count to word y of d_head and its first nhead pairs to
+ * the int32 rows (y, nhead) and then the float rows (y, nhead) that follow
+ * the nspec counts there: nspec * (1 + 2 * nhead) words, one copy to the
+ * host.  Lists past a count are left as they were.  work must hold the sum of
+ * psx_find_peaks_work_bytes over the spectra. */
+enum { PSX_PEAK_SPECTRA = 8 };
+int psx_find_peaks_spectra(const float* const* spectra, const int64_t* start, const int64_t* end, uint32_t nspec,
+                           float thr, int32_t* d_idx, float* d_snr, uint32_t cap, void* d_head, uint32_t nhead,
+                           void* work, psx_stream s);
 
 /* ------------------------------------------------------------------ */
 /* FFT (CuFFTerR2C / CuFFTerC2R, include/transforms/ffter.hpp:54-110)   */

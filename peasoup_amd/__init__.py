@@ -86,6 +86,7 @@ def lib():
         "psx_harmonic_sum": (i32, [vp, C.POINTER(vp), u32, u64, vp]),
         "psx_find_peaks_work_bytes": (u64, [u64]),
         "psx_find_peaks": (i32, [vp, i64, i64, f32, vp, vp, u32, vp, vp, vp]),
+        "psx_find_peaks_spectra": (i32, [vp, vp, vp, u32, f32, vp, vp, u32, vp, u32, vp, vp]),
         "psx_fft_plan_create": (i32, [u64, i32, u32, C.POINTER(vp)]),
         "psx_fft_plan_create_decomp": (i32, [u64, i32, u32, i32, C.POINTER(i32), C.POINTER(i32), C.POINTER(vp)]),
         "psx_fft_plan_destroy": (i32, [vp]),

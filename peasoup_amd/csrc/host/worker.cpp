@@ -87,8 +87,7 @@ void run_worker(const psx_search_args& args, DispersionTrials<float>& trials, co
         stats::normalise(pspec.get_data(), mean * size, std * size, size / 2 + 1);
         harm_folder.fold(pspec);
         SpectrumCandidates trial_cands(tim.get_dm(), (int)ii, acc_list[jj]);
-        cand_finder.find_candidates(pspec, trial_cands);
-        cand_finder.find_candidates(sums, trial_cands);
+        cand_finder.find_candidates(pspec, sums, trial_cands);
         accel_trial_cands.append(harm_finder.distill(trial_cands.cands));
       }
       auto t2 = clk::now();

@@ -430,7 +430,10 @@ void launch_harmonic(const float* P, const FoldPtrs& fp, uint64_t nb, hipStream_
 // so for the total).  Survivors are rare: the counting pass streams (16 bins
 // per thread, all four loads in flight), and almost every workgroup of the
 // writing pass ends at its count.  4.2 M bins: 7.1 + 8.3 us (one bin per load,
-// every workgroup summing counts) -> 4.8 + 4.1 us.
+// every workgroup summing counts) -> 4.8 + 4.1 us.  A trial's five spectra go
+// through one pair of launches (blockIdx.y: the spectrum): at 2^20 samples
+// 5 x (3.4 + 2.7) us -> 4.1 + 3.7 us, and their counts and first pairs come
+// back in one copy instead of up to three per spectrum.
 constexpr unsigned kPeakTile = kBlock * 16;
 typedef float psx_f4u __attribute__((ext_vector_type(4), aligned(4)));
 
@@ -449,8 +452,36 @@ __device__ inline void peak_load(const float* tile, int64_t n, unsigned r, float
   for (int j = 0; j < 4; ++j) hit[j] = at + j < n && v[j] > thr;
 }
 
-__global__ void __launch_bounds__(kBlock) k_peak_count(const float* __restrict__ p, int64_t start, int64_t end,
-                                                       float thr, uint32_t* __restrict__ counts) {
+// One spectrum alone has kernels of its own (NS = 1): with the arguments and
+// the head of several, its pair of launches took 0.8 us more at 2^23 samples.
+constexpr unsigned kPeakSpectra = PSX_PEAK_SPECTRA;
+template <unsigned NS>
+struct PeakJobs {
+  const float* p[NS];
+  int64_t start[NS], end[NS];
+  uint32_t tiles[NS];
+  uint32_t first[NS];  // first tile's place in the counts
+};
+// Pair i of spectrum y: lists idx and snr at y*cap + i (i < cap) and, where
+// asked for, hidx and hsnr at y*nhead + i (i < nhead).
+struct PeakOut {
+  int32_t* idx;
+  float* snr;
+  uint32_t cap;
+  uint32_t* total;
+  int32_t* hidx;
+  float* hsnr;
+  uint32_t nhead;
+};
+
+template <unsigned NS>
+__global__ void __launch_bounds__(kBlock) k_peak_count(const PeakJobs<NS> jobs, float thr,
+                                                       uint32_t* __restrict__ all) {
+  const unsigned y = NS == 1 ? 0 : blockIdx.y;
+  if (blockIdx.x >= jobs.tiles[y]) return;
+  const float* __restrict__ p = jobs.p[y];
+  const int64_t start = jobs.start[y], end = jobs.end[y];
+  uint32_t* __restrict__ counts = all + jobs.first[y];
   const int64_t base = start + (int64_t)blockIdx.x * kPeakTile;
   const int64_t n = min(end - base, (int64_t)kPeakTile);
   unsigned c = 0;
@@ -473,11 +504,16 @@ __global__ void __launch_bounds__(kBlock) k_peak_count(const float* __restrict__
   }
 }
 
-__global__ void __launch_bounds__(kBlock) k_peak_write(const float* __restrict__ p, int64_t start, int64_t end,
-                                                       float thr, const uint32_t* __restrict__ counts,
-                                                       unsigned ntiles, int32_t* __restrict__ oidx,
-                                                       float* __restrict__ osnr, uint32_t cap,
-                                                       uint32_t* __restrict__ total) {
+template <unsigned NS>
+__global__ void __launch_bounds__(kBlock) k_peak_write(const PeakJobs<NS> jobs, float thr,
+                                                       const uint32_t* __restrict__ all, const PeakOut out) {
+  const unsigned y = NS == 1 ? 0 : blockIdx.y;
+  const unsigned ntiles = jobs.tiles[y];
+  if (blockIdx.x >= ntiles) {
+    if (ntiles == 0 && blockIdx.x == 0 && threadIdx.x == 0) out.total[y] = 0;
+    return;
+  }
+  const uint32_t* __restrict__ counts = all + jobs.first[y];
   const unsigned mine = counts[blockIdx.x];
   const bool last = blockIdx.x == ntiles - 1;
   if (mine == 0 && !last) return;
@@ -494,8 +530,10 @@ __global__ void __launch_bounds__(kBlock) k_peak_write(const float* __restrict__
   unsigned offset = 0;
 #pragma unroll
   for (unsigned w = 0; w < kBlock / 64; ++w) offset += wave_cnt[w];
-  if (last && threadIdx.x == 0) *total = offset + mine;
+  if (last && threadIdx.x == 0) out.total[y] = offset + mine;
   if (mine == 0) return;
+  const float* __restrict__ p = jobs.p[y];
+  const int64_t start = jobs.start[y], end = jobs.end[y];
   const int64_t base = start + (int64_t)blockIdx.x * kPeakTile;
   const int64_t n = min(end - base, (int64_t)kPeakTile);
   for (unsigned r = 0; r < kPeakTile / (4 * kBlock); ++r) {
@@ -522,17 +560,18 @@ __global__ void __launch_bounds__(kBlock) k_peak_write(const float* __restrict__
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       if (hit[j]) {
-        if (pos < cap) {
-          oidx[pos] = (int32_t)(base + 4 * (int64_t)(threadIdx.x + kBlock * r) + j);
-          osnr[pos] = v[j];
+        const int32_t idx = (int32_t)(base + 4 * (int64_t)(threadIdx.x + kBlock * r) + j);
+        if (pos < out.cap) {
+          out.idx[(uint64_t)y * out.cap + pos] = idx;
+          out.snr[(uint64_t)y * out.cap + pos] = v[j];
+        }
+        if (NS > 1 && pos < out.nhead) {
+          out.hidx[y * out.nhead + pos] = idx;
+          out.hsnr[y * out.nhead + pos] = v[j];
         }
         ++pos;
       }
   }
-}
-
-__global__ void k_set_u32(uint32_t* p, uint32_t v) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) *p = v;
 }
 
 }  // namespace
@@ -818,24 +857,54 @@ extern "C" uint64_t psx_find_peaks_work_bytes(uint64_t n) {
   return ((n + kPeakTile - 1) / kPeakTile + 1) * sizeof(uint32_t);
 }
 
+namespace {
+template <unsigned NS>
+int find_peaks(const float* const* p, const int64_t* start, const int64_t* end, uint32_t nspec, float thr,
+               const PeakOut& out, void* work, hipStream_t hs) {
+  PeakJobs<NS> jobs{};
+  uint32_t most = 1, sum = 0;
+  for (uint32_t y = 0; y < nspec; ++y) {
+    const int64_t a = std::max<int64_t>(start[y], 0);
+    const uint64_t n = end[y] > a ? (uint64_t)(end[y] - a) : 0;
+    PSX_REQUIRE(n < (1ull << 31), "psx_find_peaks: range exceeds 2^31 bins");
+    jobs.p[y] = p[y];
+    jobs.start[y] = a;
+    jobs.end[y] = a + (int64_t)n;
+    jobs.tiles[y] = (uint32_t)((n + kPeakTile - 1) / kPeakTile);
+    jobs.first[y] = sum;
+    sum += jobs.tiles[y];
+    most = std::max(most, jobs.tiles[y]);
+  }
+  uint32_t* counts = (uint32_t*)work;
+  if (sum) {
+    k_peak_count<NS><<<dim3(most, nspec), kBlock, 0, hs>>>(jobs, thr, counts);
+    PSX_CHECK_LAUNCH("k_peak_count");
+  }
+  k_peak_write<NS><<<dim3(most, nspec), kBlock, 0, hs>>>(jobs, thr, counts, out);
+  PSX_CHECK_LAUNCH("k_peak_write");
+  return psx::ok();
+}
+}  // namespace
+
 extern "C" int psx_find_peaks(const float* p, int64_t start, int64_t end, float thr, int32_t* d_idx,
                               float* d_snr, uint32_t cap, uint32_t* d_count, void* work, psx_stream s) {
   PSX_REQUIRE(p && d_count && work, "psx_find_peaks: null pointer");
   PSX_REQUIRE(cap == 0 || (d_idx && d_snr), "psx_find_peaks: null output arrays");
-  if (start < 0) start = 0;
-  const hipStream_t hs = as_stream(s);
-  if (end <= start) {
-    k_set_u32<<<1, 64, 0, hs>>>(d_count, 0u);
-    PSX_CHECK_LAUNCH("k_set_u32");
-    return psx::ok();
-  }
-  const uint64_t n = (uint64_t)(end - start);
-  PSX_REQUIRE(n < (1ull << 31), "psx_find_peaks: range exceeds 2^31 bins");
-  const unsigned ntiles = (unsigned)((n + kPeakTile - 1) / kPeakTile);
-  uint32_t* counts = (uint32_t*)work;
-  k_peak_count<<<ntiles, kBlock, 0, hs>>>(p, start, end, thr, counts);
-  PSX_CHECK_LAUNCH("k_peak_count");
-  k_peak_write<<<ntiles, kBlock, 0, hs>>>(p, start, end, thr, counts, ntiles, d_idx, d_snr, cap, d_count);
-  PSX_CHECK_LAUNCH("k_peak_write");
-  return psx::ok();
+  return find_peaks<1>(&p, &start, &end, 1, thr, PeakOut{d_idx, d_snr, cap, d_count, nullptr, nullptr, 0}, work,
+                       as_stream(s));
+}
+
+extern "C" int psx_find_peaks_spectra(const float* const* spectra, const int64_t* start, const int64_t* end,
+                                      uint32_t nspec, float thr, int32_t* d_idx, float* d_snr, uint32_t cap,
+                                      void* d_head, uint32_t nhead, void* work, psx_stream s) {
+  PSX_REQUIRE(spectra && start && end && d_head && work, "psx_find_peaks_spectra: null pointer");
+  PSX_REQUIRE(nspec >= 1 && nspec <= kPeakSpectra, "psx_find_peaks_spectra: 1..%u spectra", kPeakSpectra);
+  PSX_REQUIRE(cap == 0 || (d_idx && d_snr), "psx_find_peaks_spectra: null output arrays");
+  PSX_REQUIRE(nhead <= (1u << 20), "psx_find_peaks_spectra: nhead too large");
+  for (uint32_t y = 0; y < nspec; ++y) PSX_REQUIRE(spectra[y], "psx_find_peaks_spectra: null spectrum");
+  uint32_t* head = (uint32_t*)d_head;
+  return find_peaks<kPeakSpectra>(spectra, start, end, nspec, thr,
+                                  PeakOut{d_idx, d_snr, cap, head, (int32_t*)(head + nspec),
+                                          (float*)(head + nspec + nspec * nhead), nhead},
+                                  work, as_stream(s));
 }

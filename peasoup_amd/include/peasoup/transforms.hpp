@@ -16,6 +16,7 @@
 #include <cmath>
 #include <cstdint>
 #include <cstdlib>
+#include <cstring>
 #include <fstream>
 #include <sstream>
 #include <string>
@@ -287,62 +288,99 @@ class PeakFinder {
   unsigned int max_cands;
   std::vector<int> idxs, peakidxs;
   std::vector<float> snrs, peaksnrs, peakfreqs;
+  // rows of max_cands per spectrum of a call; counts and first pairs of all
+  // its spectra, which come back in one copy
+  static constexpr unsigned int spectra = PSX_PEAK_SPECTRA, nhead = 256;
   int32_t* d_idxs = nullptr;
   float* d_snrs = nullptr;
-  uint32_t* d_count = nullptr;
+  uint32_t* d_head = nullptr;
   void* d_work = nullptr;
+  std::vector<uint32_t> head;
   psx_stream stream;
+
+  // peakfinder.hpp:77-94 for up to `spectra` spectra, in order
+  void find(DevicePowerSpectrum<float>* const* specs, unsigned int n, SpectrumCandidates& cands) {
+    peasoup::PeakWindow w[spectra];
+    const float* data[spectra];
+    int64_t start[spectra], end[spectra];
+    bool any = false;
+    for (unsigned int y = 0; y < n; ++y) {
+      w[y] = peasoup::peak_window(specs[y]->get_nbins(), specs[y]->get_bin_width(), specs[y]->get_nh(), min_freq,
+                                  max_freq);
+      data[y] = specs[y]->get_data();
+      start[y] = w[y].start;
+      end[y] = w[y].end;
+      any |= w[y].end > w[y].start;
+    }
+    std::fill(head.begin(), head.begin() + n, 0u);
+    if (any) {
+      peasoup::check(psx_find_peaks_spectra(data, start, end, n, threshold, d_idxs, d_snrs, max_cands, d_head, nhead,
+                                            d_work, stream),
+                     "Error from device_find_peaks");
+      Utils::d2hcpy(head.data(), d_head, n * (1 + 2 * nhead), stream);
+    }
+    for (unsigned int y = 0; y < n; ++y) {
+      const uint32_t c = head[y];
+      if (c > max_cands) peasoup::throw_error("PeakFinder: more than 100000 bins above threshold");
+      if (c > nhead) {
+        Utils::d2hcpy(idxs.data(), d_idxs + (std::size_t)y * max_cands, c, stream);
+        Utils::d2hcpy(snrs.data(), d_snrs + (std::size_t)y * max_cands, c, stream);
+      } else {
+        std::memcpy(idxs.data(), head.data() + n + y * nhead, c * sizeof(int));
+        std::memcpy(snrs.data(), head.data() + n + (n + y) * nhead, c * sizeof(float));
+      }
+      const int npeaks = peasoup::identify_unique_peaks(idxs.data(), snrs.data(), (int)c, min_gap, peakidxs.data(),
+                                                        peaksnrs.data());
+      for (int ii = 0; ii < npeaks; ii++) peakfreqs[ii] = peakidxs[ii] * w[y].factor;
+      cands.append(peaksnrs.data(), peakfreqs.data(), (int)specs[y]->get_nh(), npeaks);
+    }
+  }
+
+  void find_all(const std::vector<DevicePowerSpectrum<float>*>& specs, SpectrumCandidates& cands) {
+    for (std::size_t ii = 0; ii < specs.size(); ii += spectra)
+      find(&specs[ii], (unsigned int)std::min<std::size_t>(spectra, specs.size() - ii), cands);
+  }
 
  public:
   PeakFinder(float threshold, float min_freq, float max_freq, unsigned int size, int min_gap = 30,
              psx_stream s = nullptr)
       : threshold(threshold), min_freq(min_freq), max_freq(max_freq), min_gap(min_gap), max_cands(100000),
-        stream(s) {
+        head(spectra * (1 + 2 * nhead)), stream(s) {
     idxs.resize(max_cands);
     snrs.resize(max_cands);
     peakidxs.resize(max_cands);
     peaksnrs.resize(max_cands);
     peakfreqs.resize(max_cands);
-    Utils::device_malloc(&d_idxs, max_cands);
-    Utils::device_malloc(&d_snrs, max_cands);
-    Utils::device_malloc(&d_count, 1);
-    peasoup::check(psx_malloc(&d_work, psx_find_peaks_work_bytes(size / 2 + 1)), "PeakFinder");
+    Utils::device_malloc(&d_idxs, spectra * max_cands);
+    Utils::device_malloc(&d_snrs, spectra * max_cands);
+    Utils::device_malloc(&d_head, head.size());
+    peasoup::check(psx_malloc(&d_work, spectra * psx_find_peaks_work_bytes(size / 2 + 1)), "PeakFinder");
   }
   PeakFinder(const PeakFinder&) = delete;
   PeakFinder& operator=(const PeakFinder&) = delete;
   ~PeakFinder() {
     psx_free(d_idxs);
     psx_free(d_snrs);
-    psx_free(d_count);
+    psx_free(d_head);
     psx_free(d_work);
   }
 
   void find_candidates(HarmonicSums<float>& sums, SpectrumCandidates& cands) {
-    for (std::size_t ii = 0; ii < sums.size(); ii++) find_candidates(*sums[(int)ii], cands);
+    std::vector<DevicePowerSpectrum<float>*> specs;
+    for (std::size_t ii = 0; ii < sums.size(); ii++) specs.push_back(sums[(int)ii]);
+    find_all(specs, cands);
   }
 
-  // peakfinder.hpp:77-94
   void find_candidates(DevicePowerSpectrum<float>& pspec, SpectrumCandidates& cands) {
-    const peasoup::PeakWindow w =
-        peasoup::peak_window(pspec.get_nbins(), pspec.get_bin_width(), pspec.get_nh(), min_freq, max_freq);
-    int count = 0;
-    if (w.end > w.start) {
-      peasoup::check(psx_find_peaks(pspec.get_data(), w.start, w.end, threshold, d_idxs, d_snrs, max_cands, d_count,
-                                    d_work, stream),
-                     "Error from device_find_peaks");
-      uint32_t c = 0;
-      Utils::d2hcpy(&c, d_count, 1, stream);
-      if (c > max_cands) peasoup::throw_error("PeakFinder: more than 100000 bins above threshold");
-      count = (int)c;
-      if (count) {
-        Utils::d2hcpy(idxs.data(), d_idxs, count, stream);
-        Utils::d2hcpy(snrs.data(), d_snrs, count, stream);
-      }
-    }
-    const int npeaks =
-        peasoup::identify_unique_peaks(idxs.data(), snrs.data(), count, min_gap, peakidxs.data(), peaksnrs.data());
-    for (int ii = 0; ii < npeaks; ii++) peakfreqs[ii] = peakidxs[ii] * w.factor;
-    cands.append(peaksnrs.data(), peakfreqs.data(), (int)pspec.get_nh(), npeaks);
+    DevicePowerSpectrum<float>* one = &pspec;
+    find(&one, 1, cands);
+  }
+
+  // the spectrum's candidates, then its harmonic sums'
+  void find_candidates(DevicePowerSpectrum<float>& pspec, HarmonicSums<float>& sums, SpectrumCandidates& cands) {
+    std::vector<DevicePowerSpectrum<float>*> specs{&pspec};
+    for (std::size_t ii = 0; ii < sums.size(); ii++) specs.push_back(sums[(int)ii]);
+    find_all(specs, cands);
   }
 };
 

@@ -105,3 +105,41 @@ def test_c2r_pairs(psx, orc, n, batch):
     plan.execute(d_X, d_x)
     ref = np.fft.irfft(X.astype(np.complex128), n, axis=1) * n
     assert np.max(np.abs(d_x.numpy() - ref)) <= 2e-6 * np.sqrt(np.mean(ref ** 2)) * np.log2(n)
+
+
+@pytest.mark.parametrize("ranges,thr,cap,nhead", [
+    ([(0, 4097), (3, 3), (7, 100003), (100002, 100003), (0, 4096)], 2.0, 500, 16),
+    ([(0, 100003)] * 8, 0.0, 70000, 300), ([(5, 5), (9, 2)], 0.0, 10, 4), ([(13, 60001)], 3.0, 0, 1000),
+    ([(0, 1), (4095, 8193)], -9.0, 5000, 0),
+])
+def test_peaks_of_several_spectra(psx, ranges, thr, cap, nhead):
+    n = len(ranges)
+    ps = [np.random.default_rng(y).standard_normal(100003).astype(f32) for y in range(n)]
+    d_ps = [dev(psx, p) for p in ps]
+    d_i, d_s = dev(psx, np.full(n * cap + 1, -7, np.int32)), dev(psx, np.full(n * cap + 1, -7, f32))
+    d_h = dev(psx, np.full(n * (1 + 2 * nhead) + 1, 0xC0E00000, np.uint32))  # -7.0f
+    work = psx.DeviceArray(sum(int(psx.lib().psx_find_peaks_work_bytes(max(b - a, 0))) for a, b in ranges), np.uint8)
+    a64 = lambda k: (C.c_int64 * n)(*[r[k] for r in ranges])
+    psx.check(psx.lib().psx_find_peaks_spectra((C.c_void_p * n)(*[d.ptr for d in d_ps]), a64(0), a64(1), n, thr,
+                                               d_i.ptr, d_s.ptr, cap, d_h.ptr, nhead, work.ptr, None))
+    idx, snr, head = d_i.numpy(), d_s.numpy(), d_h.numpy()
+    assert idx[-1] == -7 and snr[-1] == -7 and head[-1] == 0xC0E00000
+    hidx = head[n:n + n * nhead].view(np.int32).reshape(n, nhead)
+    hsnr = head[n + n * nhead:-1].view(f32).reshape(n, nhead)
+    for y, (a, b) in enumerate(ranges):
+        want = np.flatnonzero(ps[y][a:b] > f32(thr)) + a
+        assert head[y] == want.size
+        m = min(cap, want.size)
+        assert np.array_equal(idx[y * cap:y * cap + m], want[:m]) and np.all(idx[y * cap + m:(y + 1) * cap] == -7)
+        assert np.array_equal(snr[y * cap:y * cap + m], ps[y][want[:m]])
+        m = min(nhead, want.size)
+        assert np.array_equal(hidx[y, :m], want[:m]) and np.array_equal(hsnr[y, :m], ps[y][want[:m]])
+        assert np.all(hsnr[y, m:] == -7)
+
+
+def test_peaks_of_several_spectra_refusals(psx):
+    d = dev(psx, np.zeros(64, f32))
+    ptr, at = (C.c_void_p * 9)(*[d.ptr] * 9), (C.c_int64 * 9)()
+    call = lambda n, i, h: psx.lib().psx_find_peaks_spectra(ptr, at, at, n, 0.0, i, i, 1, h, 1, d.ptr, None)
+    assert call(0, d.ptr, d.ptr) != 0 and call(9, d.ptr, d.ptr) != 0
+    assert call(1, None, d.ptr) != 0 and call(1, d.ptr, None) != 0
