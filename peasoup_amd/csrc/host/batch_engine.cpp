@@ -48,7 +48,8 @@ uint64_t Engine::device_bytes(uint64_t N, uint32_t B, uint32_t cap) {
   uint64_t b = 0;
   b += 2 * M * B * sizeof(float2);      // FFT work + Z
   b += (pst * B + kHarmWaveBins) * sizeof(float);  // P
-  b += (uint64_t)bound_stride((int64_t)pst) * B * sizeof(uint16_t);  // Q
+  // Q; its slack beyond this is part of the prologue's reserve
+  b += (uint64_t)((pst + 512) / 2 + 64) * B * sizeof(uint16_t);
   b += 2 * (uint64_t)cap * sizeof(Cand16);
   b += prologue_bytes(M);
   return b;
