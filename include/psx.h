@@ -310,7 +310,9 @@ int psx_batch_search(const psx_search_args* args, const psx_batch_opts* opts, co
                      uint32_t naccs, psx_candidate* out, uint32_t cap, uint32_t* count, double* seconds);
 
 /* Frees the engine a psx_batch_search call with keep_engine left behind
- * (its device buffers, FFT plans and launch graphs; one engine is kept per
+ * (its device buffers, FFT plans and launch graphs, and the call's dereddened
+ * series where they take no more device memory than the engine; a call that
+ * builds another engine frees those series first; one engine is kept per
  * process, replaced by the next keeping call with other arguments).  No
  * counterpart in the reference, whose Worker builds its transforms per DM
  * (pipeline_multi.cu:111-145); for pipelines that search many segments of
@@ -395,7 +397,9 @@ typedef struct psx_request_status {
 } psx_request_status;
 
 typedef struct psx_server_stats {
-  uint64_t used_bytes, budget_bytes;
+  uint64_t used_bytes, budget_bytes; /* used: engines and admitted requests; the series buffer of each
+                                        engine's last request, kept for its next, comes on top, within
+                                        the budget */
   uint32_t waiting, active, engines;
   uint64_t completed, failed, trials_done;
 } psx_server_counters;

@@ -17,7 +17,8 @@
 //             with trials waiting (PSX_DISPATCH_MIXED_GRAPH);
 //   collect   routes finished trials back to their requests; a request whose
 //             trials are all done gets the Worker's per-DM
-//             AccelerationDistiller, releases its memory and is completed.
+//             AccelerationDistiller, leaves its series buffer to the engine
+//             or frees it, and is completed.
 // Each trial's arithmetic does not depend on which batch carries it, so a
 // request's candidates are the same alone and in the mix.
 #include <hip/hip_runtime.h>
@@ -99,6 +100,11 @@ struct EngineState {
   hipStream_t stream = nullptr;
   hipEvent_t mark = nullptr;  // the engine stream's work so far (mixed dispatch waits on it)
   uint64_t bytes = 0;
+  // the series buffer of the engine's last finished request, for its next one
+  // of that size: hipFree waits for the device (0.25 ms on average, up to
+  // 5 ms, while the other engines' next batches waited to be launched)
+  float* spare = nullptr;
+  uint64_t spare_bytes = 0;
   std::deque<TrialRef> queue;        // trials waiting for a batch
   std::deque<std::vector<TrialRef>> inflight;  // trials of each submitted batch
   clk::time_point last_used;
@@ -149,7 +155,9 @@ struct psx_server {
   // combination of (engine, slot, batch size) launched so far
   hipStream_t mixed_stream = nullptr;
   std::map<std::vector<std::tuple<EngineState*, int, uint32_t>>, hipGraphExec_t> mixed_graphs;
-  uint64_t used = 0;
+  uint64_t used = 0;   // engines and admitted requests
+  uint64_t spare = 0;  // spare series buffers, freed before anything is refused or evicted for them
+  std::atomic<int> callers{0};  // API calls on their way into mu
   uint64_t completed = 0, failed = 0, trials_done = 0;
   int device = 0;
 
@@ -164,6 +172,7 @@ struct psx_server {
   void fail_request(Request* r, int code, const std::string& msg);
   EngineState* engine_for(const psx_search_args& a, bool create, uint64_t* need);
   void evict_idle(uint64_t need);
+  void drop_spares();
   bool dispatch_mixed();
   void drop_mixed_graphs(const EngineState* es);
 };
@@ -226,12 +235,24 @@ void psx_server::evict_idle(uint64_t need) {
     }
     if (victim == engines.end()) return;
     used -= victim->second->bytes;
+    spare -= victim->second->spare_bytes;
+    (void)hipFree(victim->second->spare);
     drop_mixed_graphs(victim->second.get());
     victim->second->eng.reset();
     (void)hipStreamDestroy(victim->second->stream);
     (void)hipEventDestroy(victim->second->mark);
     engines.erase(victim);
   }
+}
+
+void psx_server::drop_spares() {
+  for (auto& kv : engines) {
+    EngineState* e = kv.second.get();
+    (void)hipFree(e->spare);
+    e->spare = nullptr;
+    e->spare_bytes = 0;
+  }
+  spare = 0;
 }
 
 void psx_server::drop_mixed_graphs(const EngineState* es) {
@@ -327,16 +348,33 @@ bool psx_server::admit_one(Request* r) {
   uint64_t need_engine = 0;
   engine_for(r->spec.args, false, &need_engine);
   const uint64_t need = r->bytes + need_engine;
+  // a spare buffer of the request's own size is already part of its need
+  const EngineState* own = engine_for(r->spec.args, false, nullptr);
+  const uint64_t fits = own && own->spare_bytes == r->bytes ? r->bytes : 0;
+  if (used + spare - fits + need > cfg.hbm_budget_bytes) drop_spares();
   if (used + need > cfg.hbm_budget_bytes) evict_idle(need);
   if (used + need > cfg.hbm_budget_bytes) return false;
+  if (need_engine) drop_spares();  // an engine is built in the memory it was built in without spares
   EngineState* es = engine_for(r->spec.args, true, nullptr);
   r->es = es;
   const psx_search_args& a = r->spec.args;
   const uint64_t N = a.size;
-  if (hipMalloc(&r->d_tims, r->bytes) != hipSuccess) {
-    (void)hipGetLastError();
-    r->d_tims = nullptr;
-    return false;
+  if (es->spare_bytes == r->bytes) {
+    r->d_tims = es->spare;
+    spare -= es->spare_bytes;
+    es->spare = nullptr;
+    es->spare_bytes = 0;
+  } else {
+    hipError_t e = hipMalloc(&r->d_tims, r->bytes);
+    if (e != hipSuccess && spare) {
+      drop_spares();
+      e = hipMalloc(&r->d_tims, r->bytes);
+    }
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      r->d_tims = nullptr;
+      return false;
+    }
   }
   used += r->bytes;
   r->t_admit = now_s();
@@ -417,6 +455,14 @@ void psx_server::finish(Request* r) {
   psx::search::flatten(flat, r->result.data(), (uint32_t)r->result.size(), &cnt);
   r->per_trial.clear();
   r->zap.reset();
+  // every trial that read the series has been collected; the larger of two
+  // buffers stays with the engine
+  EngineState* es = r->es;
+  if (es->spare_bytes < r->bytes) {
+    std::swap(es->spare, r->d_tims);
+    spare += r->bytes - es->spare_bytes;
+    es->spare_bytes = r->bytes;
+  }
   (void)hipFree(r->d_tims);
   r->d_tims = nullptr;
   used -= r->bytes;
@@ -432,12 +478,20 @@ void psx_server::loop() {
   std::vector<std::vector<Candidate>> got;
   while (true) {
     bool progressed = false;
+    // let callers in: this thread releases mu for an instant only, and with
+    // work in flight a submit waited until the device had none left
+    for (int i = 0; i < 100 && callers.load() > 0; ++i) std::this_thread::yield();
     {
       std::unique_lock<std::mutex> lk(mu);
       if (stop && waiting.empty() && active.empty()) break;
+      const uint64_t ended = completed + failed;
       // admission, in arrival order (a request that does not fit blocks
-      // later ones: no starvation of large requests)
-      while (!waiting.empty() && (cfg.max_active == 0 || active.size() < cfg.max_active)) {
+      // later ones: no starvation of large requests); one at a time, so that
+      // its trials run during the next one's prologues, but for mixed
+      // batches, which take trials of all
+      bool admitted = false;
+      while (!waiting.empty() && (cfg.max_active == 0 || active.size() < cfg.max_active) &&
+             !(admitted && cfg.dispatch == PSX_DISPATCH_STREAMS)) {
         Request* r = waiting.front();
         bool ok;
         try {
@@ -449,7 +503,7 @@ void psx_server::loop() {
         }
         if (!ok) break;
         waiting.pop_front();
-        progressed = true;
+        admitted = progressed = true;
       }
       try {
         if (cfg.dispatch == PSX_DISPATCH_MIXED_GRAPH)
@@ -495,8 +549,8 @@ void psx_server::loop() {
           kv.second->inflight.clear();
         }
       }
-      cv.notify_all();
-      if (!progressed) cv.wait_for(lk, std::chrono::microseconds(200));
+      if (completed + failed != ended) cv.notify_all();
+      if (!progressed) cv.wait_for(lk, std::chrono::microseconds(active.empty() ? 200 : 50));
     }
   }
 }
@@ -534,6 +588,18 @@ extern "C" int psx_server_create(const psx_server_config* cfg, psx_server** out)
   return psx::ok();
 }
 
+// A caller's lock on the server's state; the scheduler stands back for it.
+namespace {
+struct Entry {
+  std::unique_lock<std::mutex> lk;
+  explicit Entry(psx_server* s) {
+    s->callers.fetch_add(1);
+    lk = std::unique_lock<std::mutex>(s->mu);
+    s->callers.fetch_sub(1);
+  }
+};
+}  // namespace
+
 extern "C" int psx_server_submit(psx_server* s, const psx_request* req, uint64_t* id) {
   PSX_REQUIRE(s && req && id, "psx_server_submit: null argument");
   int rc = psx::search::validate_args(&req->args);
@@ -554,7 +620,7 @@ extern "C" int psx_server_submit(psx_server* s, const psx_request* req, uint64_t
   r->spec.args.birdie_freq = r->spec.args.birdie_width = nullptr;  // the caller's arrays are not kept
   r->bytes = request_bytes(*req);
   r->t_submit = now_s();
-  std::lock_guard<std::mutex> lk(s->mu);
+  Entry entry(s);
   if (s->stop) return psx::fail(PSX_ERR_STATE, "psx_server_submit: server is shutting down");
   r->id = s->next_id++;
   *id = r->id;
@@ -576,7 +642,7 @@ static void fill_status(const Request* r, psx_request_status* st) {
 
 extern "C" int psx_server_poll(psx_server* s, uint64_t id, psx_request_status* st) {
   PSX_REQUIRE(s && st, "psx_server_poll: null argument");
-  std::lock_guard<std::mutex> lk(s->mu);
+  Entry entry(s);
   auto it = s->all.find(id);
   PSX_REQUIRE(it != s->all.end(), "psx_server_poll: unknown request %llu", (unsigned long long)id);
   fill_status(it->second.get(), st);
@@ -585,7 +651,8 @@ extern "C" int psx_server_poll(psx_server* s, uint64_t id, psx_request_status* s
 
 extern "C" int psx_server_wait(psx_server* s, uint64_t id, double timeout_s, psx_request_status* st) {
   PSX_REQUIRE(s && st, "psx_server_wait: null argument");
-  std::unique_lock<std::mutex> lk(s->mu);
+  Entry entry(s);
+  std::unique_lock<std::mutex>& lk = entry.lk;
   auto it = s->all.find(id);
   PSX_REQUIRE(it != s->all.end(), "psx_server_wait: unknown request %llu", (unsigned long long)id);
   Request* r = it->second.get();
@@ -604,7 +671,7 @@ extern "C" int psx_server_wait(psx_server* s, uint64_t id, double timeout_s, psx
 
 extern "C" int psx_server_result(psx_server* s, uint64_t id, psx_candidate* out, uint32_t cap, uint32_t* count) {
   PSX_REQUIRE(s && count, "psx_server_result: null argument");
-  std::lock_guard<std::mutex> lk(s->mu);
+  Entry entry(s);
   auto it = s->all.find(id);
   PSX_REQUIRE(it != s->all.end(), "psx_server_result: unknown request %llu", (unsigned long long)id);
   Request* r = it->second.get();
@@ -620,7 +687,7 @@ extern "C" int psx_server_result(psx_server* s, uint64_t id, psx_candidate* out,
 
 extern "C" int psx_server_stats(psx_server* s, psx_server_counters* st) {
   PSX_REQUIRE(s && st, "psx_server_stats: null argument");
-  std::lock_guard<std::mutex> lk(s->mu);
+  Entry entry(s);
   st->used_bytes = s->used;
   st->budget_bytes = s->cfg.hbm_budget_bytes;
   st->waiting = (uint32_t)s->waiting.size();
@@ -642,6 +709,7 @@ extern "C" int psx_server_destroy(psx_server* s) {
   if (s->sched.joinable()) s->sched.join();
   if (s->mixed_stream) (void)hipStreamSynchronize(s->mixed_stream);
   for (auto& g : s->mixed_graphs) (void)hipGraphExecDestroy(g.second);
+  s->drop_spares();
   for (auto& kv : s->engines) {
     kv.second->eng.reset();
     (void)hipStreamDestroy(kv.second->stream);

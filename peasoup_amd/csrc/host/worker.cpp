@@ -26,14 +26,15 @@ struct Timings {
   double prologue = 0, accel = 0, distill = 0;
 };
 
-// pipeline_multi.cu:111-303 for the DM indices of `trials`.
-void run_worker(const psx_search_args& args, DispersionTrials<float>& trials, const float* accs, uint32_t naccs,
-                CandidateCollection& dm_trial_cands, Timings& tm) {
+// pipeline_multi.cu:111-303 for the series (nsamps samples each) of dm_list,
+// read where the caller has them: DispersionTrials would hold a copy.
+void run_worker(const psx_search_args& args, const float* series, uint64_t nsamps, const std::vector<float>& dm_list,
+                const float* accs, uint32_t naccs, CandidateCollection& dm_trial_cands, Timings& tm) {
   const unsigned int size = (unsigned int)args.size;
-  const bool padding = size > trials.get_nsamps();
+  const bool padding = size > nsamps;
   CuFFTerR2C r2cfft(size);
   CuFFTerC2R c2rfft(size);
-  const float tobs = size * trials.get_tsamp();
+  const float tobs = size * args.tsamp;
   const float bin_width = 1.0 / tobs;
   DeviceFourierSeries<psx_c32> d_fseries(size / 2 + 1, bin_width);
   DedispersedTimeSeries<float> tim;
@@ -58,13 +59,16 @@ void run_worker(const psx_search_args& args, DispersionTrials<float>& trials, co
   peasoup::check(psx_malloc(&stats_work, psx_reduce_work_bytes()), "Worker");
   float mean, std, rms;
   try {
-    for (std::size_t ii = 0; ii < trials.get_count(); ++ii) {
+    for (std::size_t ii = 0; ii < dm_list.size(); ++ii) {
       psx::TraceRange dm_range("DM-Loop");
       auto t0 = clk::now();
-      trials.get_idx(ii, tim, size);
+      tim.set_data(const_cast<float*>(series) + ii * nsamps);  // only read
+      tim.set_dm(dm_list[ii]);
+      tim.set_nsamps(nsamps);
+      tim.set_tsamp(args.tsamp);
       d_tim.copy_from_host(tim);
       d_tim.remove_baseline(std::min(tim.get_nsamps(), d_tim.get_nsamps()));
-      if (padding && tim.get_nsamps() < d_tim.get_nsamps()) d_tim.fill(trials.get_nsamps(), d_tim.get_nsamps(), 0);
+      if (padding && tim.get_nsamps() < d_tim.get_nsamps()) d_tim.fill(nsamps, d_tim.get_nsamps(), 0);
       if (accs)
         acc_list.assign(accs, accs + naccs);
       else
@@ -130,12 +134,9 @@ extern "C" int psx_worker_search(const psx_search_args* args, const float* serie
   PSX_REQUIRE(series && dm_list && ndm > 0 && nsamps > 0, "psx_worker_search: bad series");
   PSX_REQUIRE(!accs || naccs > 0, "psx_worker_search: empty acceleration list");
   try {
-    DispersionTrials<float> trials(args->tsamp);
-    trials.resize(nsamps, std::vector<float>(dm_list, dm_list + ndm));
-    std::memcpy(trials.get_data_ptr(), series, sizeof(float) * nsamps * ndm);
     CandidateCollection dm_trial_cands;
     Timings tm;
-    run_worker(*args, trials, accs, naccs, dm_trial_cands, tm);
+    run_worker(*args, series, nsamps, std::vector<float>(dm_list, dm_list + ndm), accs, naccs, dm_trial_cands, tm);
     if (seconds) {
       seconds[0] = tm.prologue;
       seconds[1] = tm.accel;
