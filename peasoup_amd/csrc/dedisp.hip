@@ -143,49 +143,73 @@ __global__ void __launch_bounds__(kB) k_unpack_t(const uint8_t* __restrict__ in,
 
 // --------------------------------------------------------------------- sum
 // out[dm][t] = sum_c row_c[t + delay(dm, c)] / denom over tiles of 1,024
-// samples, kDms DM trials per wave.  Samples are added as packed 16-bit pairs
-// (even and odd bytes of a dword); up to 4 bits four channels are first added
-// as packed bytes (4 x 15 < 256).  The pairs hold 65535: WIDE sums (channels *
-// the largest sample above that) spill them into 32-bit sums every kFlush
-// channels.  All sums are exact integers.
+// samples, kDms DM trials per wave.  Samples are added four to a dword.  Up to
+// 4 bits a run of channels is added as packed bytes (16 x 15, 84 x 3 and
+// 252 x 1 fit), then as pairs; 8-bit samples go to the pairs at once.  Of the
+// two pairs of 16-bit sums only the odd bytes' one is kept (hi); beside it the
+// plain sum of the dwords mod 2^32 (lo), which is the even bytes' pair plus
+// 2^8 times the odd bytes' one.  That takes 4 instructions per 8 samples at 8
+// bits (6 with both pairs masked out of each dword) and 2 per 16 up to 4 bits.
+// The pairs hold 65535: WIDE sums (channels * the largest sample above that)
+// spill them into 32-bit sums every kFlush channels.  All sums are exact
+// integers.
 constexpr int kDms = 4;             // DM trials per wave
 constexpr int kTileSamps = 1024;    // samples per wave: four dwords per lane
 
 template <int NBITS, bool WIDE>
 struct DmSums {
   static constexpr uint32_t kFlush = NBITS == 8 ? 256 : 4096;  // kFlush * (2^NBITS - 1) <= 65535
-  uint32_t lo[4], hi[4];         // samples 4q, 4q+2 and 4q+1, 4q+3
+  // channels per run: as many as four packed bytes hold (a multiple of 4)
+  static constexpr uint32_t kRun = NBITS == 8 ? kFlush : 255 / ((1 << NBITS) - 1) / 4 * 4;
+  uint32_t lo[4], hi[4];  // packed dwords (mod 2^32); samples 4q+1, 4q+3 as pairs
+  uint32_t run[NBITS == 8 ? 1 : 4];
   uint32_t sum[WIDE ? 16 : 1];
   __device__ void clear() {
 #pragma unroll
     for (int q = 0; q < 4; ++q) lo[q] = hi[q] = 0u;
+    if constexpr (NBITS < 8) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) run[q] = 0u;
+    }
     if constexpr (WIDE) {
 #pragma unroll
       for (int q = 0; q < 16; ++q) sum[q] = 0u;
     }
   }
-  __device__ static uint32_t even(uint32_t x) { return x & 0x00FF00FFu; }
   __device__ static uint32_t odd(uint32_t x) { return __builtin_amdgcn_perm(0u, x, 0x0C030C01u); }
   // dword q of four channels
   __device__ void add4(int q, uint32_t x0, uint32_t x1, uint32_t x2, uint32_t x3) {
-    if constexpr (NBITS <= 4) {
-      const uint32_t s = x0 + x1 + x2 + x3;
-      lo[q] += even(s);
-      hi[q] += odd(s);
+    if constexpr (NBITS < 8) {
+      run[q] = run[q] + x0 + x1;
+      run[q] = run[q] + x2 + x3;
     } else {
-      lo[q] += even(x0) + even(x1);
-      hi[q] += odd(x0) + odd(x1);
-      lo[q] += even(x2) + even(x3);
-      hi[q] += odd(x2) + odd(x3);
+      lo[q] = lo[q] + x0 + x1;
+      hi[q] = hi[q] + odd(x0) + odd(x1);
+      lo[q] = lo[q] + x2 + x3;
+      hi[q] = hi[q] + odd(x2) + odd(x3);
     }
   }
+  // after at most kRun channels
+  __device__ void end_run() {
+    if constexpr (NBITS < 8) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        lo[q] += run[q];
+        hi[q] += odd(run[q]);
+        run[q] = 0u;
+      }
+    }
+  }
+  // samples 4q, 4q+2 as pairs
+  __device__ uint32_t even(int q) const { return lo[q] - (hi[q] << 8); }
+  // after at most kFlush channels
   __device__ void flush() {
     if constexpr (WIDE) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        sum[4 * q] += lo[q] & 0xFFFFu;
+        sum[4 * q] += even(q) & 0xFFFFu;
         sum[4 * q + 1] += hi[q] & 0xFFFFu;
-        sum[4 * q + 2] += lo[q] >> 16;
+        sum[4 * q + 2] += even(q) >> 16;
         sum[4 * q + 3] += hi[q] >> 16;
         lo[q] = hi[q] = 0u;
       }
@@ -193,7 +217,7 @@ struct DmSums {
   }
   __device__ uint32_t at(int q, int i) const {
     if constexpr (WIDE) return sum[4 * q + i];
-    else return i == 0 ? lo[q] & 0xFFFFu : i == 1 ? hi[q] & 0xFFFFu : i == 2 ? lo[q] >> 16 : hi[q] >> 16;
+    else return i == 0 ? even(q) & 0xFFFFu : i == 1 ? hi[q] & 0xFFFFu : i == 2 ? even(q) >> 16 : hi[q] >> 16;
   }
   // samples t .. t+3 of dword q to o (the first n of them)
   __device__ void store(int q, float denom, float* o, uint32_t n) const {
@@ -217,14 +241,18 @@ struct DmSums {
 // whole dwords of one copy, read by consecutive lanes without bank conflicts
 // (byte-shifted reads of one copy would need a shift per dword; unaligned
 // 16-byte loads straight from the rows take 6.0 ms for 128 DMs x 987 8-bit
-// channels x 521k samples, this form 2.7 ms, and one byte per lane and load,
+// channels x 521k samples, this form 2.2 ms, and one byte per lane and load,
 // one DM per workgroup, took 33.5 ms).  Channels are staged four at a time,
 // double buffered: the next four are loaded into registers while the current
-// ones are summed.  Bound by the packed adds (6 instructions per 8 samples at
-// 8 bits, 6 per 16 up to 4 bits: 1.4 ms of issue for that shape) and the LDS
-// reads they wait for.
+// ones are summed.  What a stage needs of the delay table comes from LDS too,
+// filled for 64 channels at a time by all threads: with 20 scalar loads and
+// 160 scalar instructions per wave and stage, and the stage's addresses a
+// dependent load away, it took 2.6 ms.  Bound by its instructions and by the
+// waits of the stages: the adds are 55% of the vector ones (1.2 ms of issue in
+// all), staging four copies costs 0.8 ms of the 2.2, waiting for the rows 0.2.
 constexpr int kChunk = 4;             // channels per stage
-constexpr uint32_t kMaxPitch = 512;   // dwords per copy, at most: 64 KB of LDS, two workgroups per CU
+constexpr uint32_t kSpan = 64;        // channels per table
+constexpr uint32_t kMaxPitch = 512;   // dwords per copy, at most: 64 KB of LDS (and 9 of tables), two workgroups per CU
 struct SumArgs {
   const uint8_t* rows;
   uint64_t nsamps_in;
@@ -242,17 +270,36 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4)
 k_dedisp_lds(const SumArgs a, uint32_t ngroups, uint32_t nblocks) {
   using Sums = DmSums<NBITS, WIDE>;
   constexpr int kMaxTasks = (int)kMaxPitch / (64 * NW);
-  extern __shared__ uint32_t lds[];  // [2][kChunk][4][pitch]
+  extern __shared__ uint4 lds4[];
+  uint32_t* const lds = reinterpret_cast<uint32_t*>(lds4);  // [2][kChunk][4][pitch], then the tables
+  uint32_t* const area = lds + 2 * kChunk * 4 * a.pitch;
+  // of the channels of two table spans: byte offset in a stage's copies of
+  // every (channel, DM) stretch, and the first DM's delay
+  uint2* const offs = reinterpret_cast<uint2*>(area);                             // [2][kSpan/4][4*NW]
+  int32_t* const first = reinterpret_cast<int32_t*>(area + 2 * kSpan * 2 * NW);  // [2*kSpan]
   const uint32_t blk = psx::xcd_logical_block(blockIdx.x, nblocks);
   const uint64_t tbase = (uint64_t)(blk / ngroups) * kTileSamps;
   const uint32_t g0 = (blk % ngroups) * (kDms * NW);  // first DM of the group
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t dm0 = g0 + wave * kDms;
-  const int32_t* first = a.delays + (uint64_t)g0 * a.nrows;
-  const int32_t* dl[kDms];
+  // one thread per DM and four channels; channels past the last one hold
+  // zeros at any offset
+  static_assert(kSpan / 4 * kDms * NW == 64 * NW, "one table entry per thread");
+  auto fill = [&](uint32_t span) {
+    const uint32_t q = threadIdx.x % (kSpan / 4), d = threadIdx.x / (kSpan / 4);
+    const int32_t* f = a.delays + (uint64_t)g0 * a.nrows;
+    const int32_t* dl = a.delays + (uint64_t)min(g0 + d, a.ndm - 1) * a.nrows;
+    uint32_t o[4];
 #pragma unroll
-  for (int k = 0; k < kDms; ++k) dl[k] = a.delays + (uint64_t)min(dm0 + (uint32_t)k, a.ndm - 1) * a.nrows;
+    for (uint32_t j = 0; j < 4; ++j) {
+      const uint32_t c = min(span * kSpan + 4 * q + j, a.nrows - 1);
+      const uint32_t rel = (uint32_t)(dl[c] - f[c]);
+      o[j] = 4u * ((4 * j + (rel & 3u)) * a.pitch + (rel >> 2));
+      if (d == 0) first[(span & 1u) * kSpan + 4 * q + j] = f[c];
+    }
+    offs[((span & 1u) * (kSpan / 4) + q) * (kDms * NW) + d] = make_uint2(o[0] | o[1] << 16, o[2] | o[3] << 16);
+  };
   const uint32_t nstep = a.pitch / 4;  // 16-byte steps of a copy
   const uint32_t ntasks = kChunk * nstep;
   uint32_t r[kMaxTasks][5];
@@ -268,7 +315,7 @@ k_dedisp_lds(const SumArgs a, uint32_t ngroups, uint32_t nblocks) {
 #pragma unroll
       for (int q = 0; q < 5; ++q) r[i][q] = 0u;
       if (task < ntasks && c < a.nrows) {
-        const uint64_t at = tbase + (uint32_t)first[c] + 16u * st;
+        const uint64_t at = tbase + (uint32_t)first[c % (2 * kSpan)] + 16u * st;
         if (at < a.nsamps_in) {
           const PSX_GLOBAL uint8_t* p = (const PSX_GLOBAL uint8_t*)(a.rows + (uint64_t)c * a.nsamps_in + at);
           const psx_u4 x = *(const PSX_GLOBAL psx_u4*)p;
@@ -302,27 +349,39 @@ k_dedisp_lds(const SumArgs a, uint32_t ngroups, uint32_t nblocks) {
   Sums acc[kDms];
 #pragma unroll
   for (int k = 0; k < kDms; ++k) acc[k].clear();
+  fill(0);
+  __syncthreads();
   load(0);
   put(0);
   __syncthreads();
-  uint32_t buf = 0;
-  const uint32_t step = WIDE ? Sums::kFlush : a.nrows;
+  uint32_t buf = 0, flushed = 0;
 #pragma unroll 1
-  for (uint32_t cs = 0; cs < a.nrows; cs += step) {
-    const uint32_t ce = min(cs + step, a.nrows);
+  for (uint32_t cs = 0; cs < a.nrows; cs += Sums::kRun) {
+    const uint32_t ce = min(cs + Sums::kRun, a.nrows);
+    if (WIDE && ce - flushed > Sums::kFlush) {
+#pragma unroll
+      for (int k = 0; k < kDms; ++k) acc[k].flush();
+      flushed = cs;
+    }
 #pragma unroll 1
     for (uint32_t c0 = cs; c0 < ce; c0 += kChunk) {
+      // the next span's entries replace those of the previous one, last read
+      // before the last barrier
+      if (c0 % kSpan == 0) fill(c0 / kSpan + 1);
+      const uint4* o4 =
+          reinterpret_cast<const uint4*>(offs + c0 % (2 * kSpan) / 4 * (kDms * NW) + wave * kDms);
+      const uint4 oa = o4[0], ob = o4[1];
+      const uint32_t o[8] = {oa.x, oa.y, oa.z, oa.w, ob.x, ob.y, ob.z, ob.w};
       load(c0 + kChunk);
-      const uint32_t* area = lds + buf * (kChunk * 4) * a.pitch + lane;
+      const uint32_t base = (buf * (kChunk * 4) * a.pitch + lane) * 4;
 #pragma unroll
       for (int k = 0; k < kDms; ++k) {
         uint32_t x[kChunk][4];
 #pragma unroll
         for (int j = 0; j < kChunk; ++j) {
-          // channels past the last one hold zeros at any offset
-          const uint32_t c = min(c0 + (uint32_t)j, a.nrows - 1);
-          const uint32_t rel = (uint32_t)(dl[k][c] - first[c]);
-          const uint32_t* p = area + (4 * j + (rel & 3u)) * a.pitch + (rel >> 2);
+          const uint32_t w = o[2 * k + j / 2];
+          const uint32_t* p =
+              reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(lds) + (base + (j & 1 ? w >> 16 : w & 0xFFFFu)));
 #pragma unroll
           for (int q = 0; q < 4; ++q) x[j][q] = p[64 * q];
         }
@@ -334,8 +393,10 @@ k_dedisp_lds(const SumArgs a, uint32_t ngroups, uint32_t nblocks) {
       buf ^= 1u;
     }
 #pragma unroll
-    for (int k = 0; k < kDms; ++k) acc[k].flush();
+    for (int k = 0; k < kDms; ++k) acc[k].end_run();
   }
+#pragma unroll
+  for (int k = 0; k < kDms; ++k) acc[k].flush();
 #pragma unroll
   for (int k = 0; k < kDms; ++k) {
     if (dm0 + (uint32_t)k >= a.ndm) continue;
@@ -377,9 +438,14 @@ __global__ void __launch_bounds__(kB) k_dedisp(const SumArgs a, uint32_t ngroups
   Sums acc[D];
 #pragma unroll
   for (int k = 0; k < D; ++k) acc[k].clear();
-  const uint32_t step = WIDE ? Sums::kFlush : a.nrows;
-  for (uint32_t cs = 0; cs < a.nrows; cs += step) {
-    const uint32_t ce = min(cs + step, a.nrows);
+  uint32_t flushed = 0;
+  for (uint32_t cs = 0; cs < a.nrows; cs += Sums::kRun) {
+    const uint32_t ce = min(cs + Sums::kRun, a.nrows);
+    if (WIDE && ce - flushed > Sums::kFlush) {
+#pragma unroll
+      for (int k = 0; k < D; ++k) acc[k].flush();
+      flushed = cs;
+    }
     uint32_t c = cs;
     for (; c + 4 <= ce; c += 4) {
 #pragma unroll
@@ -401,8 +467,10 @@ __global__ void __launch_bounds__(kB) k_dedisp(const SumArgs a, uint32_t ngroups
       }
     }
 #pragma unroll
-    for (int k = 0; k < D; ++k) acc[k].flush();
+    for (int k = 0; k < D; ++k) acc[k].end_run();
   }
+#pragma unroll
+  for (int k = 0; k < D; ++k) acc[k].flush();
 #pragma unroll
   for (int k = 0; k < D; ++k) {
     if (dm0 + (uint32_t)k >= a.ndm) continue;
@@ -443,7 +511,8 @@ int launch_lds(const SumArgs& a, hipStream_t s) {
   const uint64_t groups = (a.ndm + kDms * NW - 1) / (kDms * NW), tiles = (a.nout + kTileSamps - 1) / kTileSamps;
   PSX_REQUIRE(groups * tiles < (1ull << 31), "psx_dedisperse: too many DMs x samples");
   const uint32_t blocks = (uint32_t)(groups * tiles);
-  k_dedisp_lds<NBITS, NW, WIDE><<<blocks, 64 * NW, 2 * kChunk * 4 * a.pitch * 4, s>>>(a, (uint32_t)groups, blocks);
+  const uint32_t lds = 2 * kChunk * 4 * a.pitch * 4 + 2 * kSpan * 2 * NW * 4 + 2 * kSpan * 4;
+  k_dedisp_lds<NBITS, NW, WIDE><<<blocks, 64 * NW, lds, s>>>(a, (uint32_t)groups, blocks);
   PSX_CHECK_LAUNCH("k_dedisp_lds");
   return PSX_OK;
 }
@@ -467,13 +536,21 @@ int launch_sum(SumArgs a, const float* dm_list, float tmax, hipStream_t s) {
   constexpr bool kCanWide = (uint64_t)kMaxChans * kMax > 65535u;
   const uint64_t tiles = (a.nout + kTileSamps - 1) / kTileSamps;
   // eight waves (32 DM trials) share a staged stretch; four where eight would
-  // leave less than two workgroups per CU
-  const bool eight = a.ndm > 16 && (a.ndm + 31) / 32 * tiles >= 512;
-  a.pitch = staged_pitch(dm_list, a.ndm, eight ? 32 : 16, tmax);
+  // leave less than two workgroups per CU or where their stretch is too long
+  // for the LDS (128 DMs of 512 2-bit channels x 400k samples to DM 200:
+  // directly 2.43 ms, four waves 1.16).  Two waves hold too many of their
+  // stretch's bytes in registers and lose to the direct form (40 DMs of 512
+  // 4-bit channels to DM 250: 1.63 ms against 0.41)
+  uint32_t nw = a.ndm > 16 && (a.ndm + 31) / 32 * tiles >= 512 ? 8 : 4;
+  a.pitch = staged_pitch(dm_list, a.ndm, kDms * nw, tmax);
+  if (nw == 8 && a.pitch > kMaxPitch) {
+    nw = 4;
+    a.pitch = staged_pitch(dm_list, a.ndm, kDms * nw, tmax);
+  }
   if (a.nrows > 0 && a.ndm > 2 && a.pitch && a.pitch <= kMaxPitch) {
     if constexpr (kCanWide)
-      if (wide) return eight ? launch_lds<NBITS, 8, true>(a, s) : launch_lds<NBITS, 4, true>(a, s);
-    return eight ? launch_lds<NBITS, 8, false>(a, s) : launch_lds<NBITS, 4, false>(a, s);
+      if (wide) return nw == 8 ? launch_lds<NBITS, 8, true>(a, s) : launch_lds<NBITS, 4, true>(a, s);
+    return nw == 8 ? launch_lds<NBITS, 8, false>(a, s) : launch_lds<NBITS, 4, false>(a, s);
   }
   // four DM trials per wave share cache lines; one where four would leave the
   // chip short of waves (fewer than eight per CU)

@@ -65,3 +65,16 @@ def test_dedisperse_tiles(psx, orc, nbits, nchans, nsamps, ndm, masked, top, rea
     got = d_out.numpy()
     assert np.array_equal(got[:, :nout], ref)
     assert np.all(got[:, nout:] == -1.0)  # nothing past the output samples
+
+
+@pytest.mark.parametrize("nbits,nchans,nsamps,ndm,masked,top,reach", [
+    # runs of 16, 84 and 252 channels whose packed bytes are full, and the
+    # 64-channel spans of the staged form's tables: one less, exact, one more
+    (4, 34, 3000, 5, 1, True, 300), (4, 64, 3000, 5, 0, True, 300), (4, 66, 3000, 2, 1, True, 300),
+    (2, 88, 3000, 5, 4, True, 300), (2, 172, 3000, 7, 3, True, 300), (2, 132, 3000, 2, 3, True, 300),
+    (1, 256, 3000, 5, 4, True, 300), (1, 512, 3000, 7, 7, True, 300), (1, 264, 3000, 2, 11, True, 300),
+    (8, 63, 3000, 5, 0, True, 300), (8, 128, 3000, 19, 0, True, 300), (8, 129, 3000, 5, 0, True, 300),
+    (8, 64, 300001, 40, 1, False, 2000),     # a stretch too long for eight waves: four
+])
+def test_dedisperse_runs_and_spans(psx, orc, nbits, nchans, nsamps, ndm, masked, top, reach):
+    test_dedisperse_tiles(psx, orc, nbits, nchans, nsamps, ndm, masked, top, reach)
