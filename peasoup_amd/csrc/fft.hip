@@ -516,12 +516,11 @@ static void two_pass_tiles(Decomp& d, uint32_t batch) {
 // Default decomposition: one pass when a single-workgroup kernel exists, else
 // two passes of about equal length, the strided one the largest power of two
 // that is at most 1,024 and no longer than the contiguous last one (whose
-// rows are read and written whole).  Against the longest last pass, which
+// rows are read and written whole), but 512 for 256.  Against the longest last pass, which
 // this rule replaces below 2^23 samples (R2C of one transform and, in the
 // batched search, us per trial): 2^17 17.2 and 1.68 -> 12.7 and 0.95, 2^20
 // 21.2 and 5.10 -> 17.4 and 5.01, 2^21 31.1 and 10.93 -> 26.3 and 9.80, 3*2^17
-// 27.1 and 4.28 -> 18.6 and 2.22, 3*2^21 65.3 and 36.1 -> 52.8 and 33.2; batched
-// 3*2^20 is even (16.79, 16.87).
+// 27.1 and 4.28 -> 15.4 and 2.05, 3*2^21 65.3 and 36.1 -> 43.9 and 27.9.
 // Longer: the split with the longest last pass while the strided pass is at
 // most 2,048 points (2^24: 2,048 x 4,096), else three passes as below.
 bool default_decomp(uint64_t M, Decomp& d, uint32_t batch) {
@@ -538,8 +537,15 @@ bool default_decomp(uint64_t M, Decomp& d, uint32_t batch) {
     if (M % M2 || M1 < M2 || M1 > 4096) continue;
     if (!len_supported(M1, true) || !len_supported(M2, true)) continue;
     d.npass = 2;
-    d.L[0] = (int)M2;
-    d.L[1] = (int)M1;
+    // a strided pass of 256 points ends on radix 16, whose four-step twiddles
+    // are looked up whole: 512 points, ending on radix 2, before the half as
+    // long rows (R2C of 1, 8 and 64 transforms: 2^18 14.4, 22.9, 89 -> 13.7,
+    // 19.8, 82 us, 3*2^16 15.5, 22.8, 74 -> 14.3, 20.1, 64, 3*2^17 17.0, 28.8,
+    // 133 -> 15.4, 26.3, 131; searches in batches of 8 and 64 4% less).  At
+    // 2^17 batches of 8 lose more (6.2 -> 6.9 us per trial) than R2C gains.
+    const bool longer = M2 == 256 && M1 > 256;
+    d.L[0] = (int)(longer ? 2 * M2 : M2);
+    d.L[1] = (int)(longer ? M1 / 2 : M1);
     two_pass_tiles(d, batch);
     return pick_tiles(d);
   }
