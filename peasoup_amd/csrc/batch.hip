@@ -940,6 +940,11 @@ k_harm_bound(const float* __restrict__ P, int64_t pstride, const uint16_t* __res
       }
     };
     auto in_window = [&](uint32_t i, int k) { return (int32_t)i >= w.start[k + 1] && (int32_t)i < w.end[k + 1]; };
+    // a bin's own bound: an odd bin lies in two entries
+    auto qval = [&](uint32_t x) {
+      const float a = __uint_as_float((uint32_t)qg[x / 2] << 16), b = __uint_as_float((uint32_t)qg[(x + 1) / 2] << 16);
+      return fminf(a, b);
+    };
 #pragma unroll
     for (int d = 0; d < kBoundD; ++d) {
       uint64_t crossing = __ballot(fail[d]);
@@ -949,8 +954,17 @@ k_harm_bound(const float* __restrict__ P, int64_t pstride, const uint16_t* __res
           crossing &= crossing - 1;
           uint32_t i;
           float s;
-          pair_folds<NF>(pval, g, hi, i, s);
           const uint32_t k = lane & 31u;
+          if constexpr (NF == 5) {
+            // 32 bounds over three bins each cross for 1.7e-3 of the bins of
+            // noise (fold 4: 3e-5): first the sums of the bins' own bounds,
+            // which are no less than the exact ones, added in their order
+            // (searches of 2^24 samples with five folds 17.3 -> 15.9 ms, of
+            // 2^23 5.4 -> 5.0; no difference at four)
+            pair_folds<NF>(qval, g, hi, i, s);
+            if (__ballot(k < NF && i < hi && s > w.thr) == 0) continue;
+          }
+          pair_folds<NF>(pval, g, hi, i, s);
           bool in = false;
 #pragma unroll
           for (int f = 0; f < NF; ++f) in |= k == (uint32_t)f && in_window(i, f);
