@@ -857,8 +857,12 @@ __device__ inline void pair_folds(F f, uint32_t g, uint32_t hi, uint32_t& i, flo
   }
 }
 // Pairs of one lane row (d) up to which the wave takes them one after the
-// other; where more cross (thresholds inside the noise) each lane sums its own.
-constexpr int kSerialPairs = 8;
+// other; where more cross (thresholds inside the noise) each lane sums its own,
+// first from the bins' own bounds.  (Searches of 2^23 samples, 64 trials, five
+// folds at S/N 5.5: 8 pairs and no own bounds 21.7 ms, with them 15.6, 24 pairs
+// 12.7; at S/N 5 114, 104, 98.)
+template <int NF>
+constexpr int kSerialPairs = NF == 5 ? 24 : 8;
 
 template <int NF, bool FROM_ROWS>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NF <= 4 ? 4 : 2)))
@@ -948,14 +952,30 @@ k_harm_bound(const float* __restrict__ P, int64_t pstride, const uint16_t* __res
 #pragma unroll
     for (int d = 0; d < kBoundD; ++d) {
       uint64_t crossing = __ballot(fail[d]);
-      if (__popcll(crossing) <= kSerialPairs) {
+      bool refined = false;
+      if (__popcll(crossing) > kSerialPairs<NF>) {
+        refined = true;
+        // each lane sums its pair again from the bins' own bounds
+        bool still = false;
+#pragma unroll 1
+        for (uint32_t b = 0; b < 2; ++b) {
+          const uint32_t i = 2 * (g0 + 64u * (uint32_t)d) + b;
+          float s[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+          if (fail[d] && i < hi) harmonic_sums_rolled<NF>(qval, i, s);
+#pragma unroll
+          for (int k = 0; k < NF; ++k) still |= s[k] > w.thr;
+        }
+        fail[d] = fail[d] && still;
+        crossing = __ballot(fail[d]);
+      }
+      if (__popcll(crossing) <= kSerialPairs<NF>) {
         while (crossing) {
           const uint32_t g = base + 64u * (uint32_t)d + (uint32_t)__builtin_ctzll(crossing);
           crossing &= crossing - 1;
           uint32_t i;
           float s;
           const uint32_t k = lane & 31u;
-          if constexpr (NF == 5) {
+          if (NF == 5 && !refined) {
             // 32 bounds over three bins each cross for 1.7e-3 of the bins of
             // noise (fold 4: 3e-5): first the sums of the bins' own bounds,
             // which are no less than the exact ones, added in their order
