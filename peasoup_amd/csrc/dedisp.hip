@@ -380,8 +380,8 @@ k_dedisp_lds(const SumArgs a, uint32_t ngroups, uint32_t nblocks) {
 #pragma unroll
         for (int j = 0; j < kChunk; ++j) {
           const uint32_t w = o[2 * k + j / 2];
-          const uint32_t* p =
-              reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(lds) + (base + (j & 1 ? w >> 16 : w & 0xFFFFu)));
+          const uint32_t at = base + (j & 1 ? w >> 16 : w & 0xFFFFu);
+          const uint32_t* p = reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(lds) + at);
 #pragma unroll
           for (int q = 0; q < 4; ++q) x[j][q] = p[64 * q];
         }
@@ -512,6 +512,9 @@ int launch_lds(const SumArgs& a, hipStream_t s) {
   PSX_REQUIRE(groups * tiles < (1ull << 31), "psx_dedisperse: too many DMs x samples");
   const uint32_t blocks = (uint32_t)(groups * tiles);
   const uint32_t lds = 2 * kChunk * 4 * a.pitch * 4 + 2 * kSpan * 2 * NW * 4 + 2 * kSpan * 4;
+  if (lds > 65536)
+    PSX_CHECK_HIP(hipFuncSetAttribute((const void*)&k_dedisp_lds<NBITS, NW, WIDE>,
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   k_dedisp_lds<NBITS, NW, WIDE><<<blocks, 64 * NW, lds, s>>>(a, (uint32_t)groups, blocks);
   PSX_CHECK_LAUNCH("k_dedisp_lds");
   return PSX_OK;

@@ -208,8 +208,8 @@ struct KeptEngine {
   hipStream_t s = nullptr;
   EngineKey key;
   void reset() {
+    eng.reset();  // waits for the batch stream, which reads the series
     buf.reset();
-    eng.reset();
     if (s) (void)hipStreamDestroy(s);
     s = nullptr;
   }
@@ -376,11 +376,18 @@ extern "C" int psx_batch_search(const psx_search_args* args, const psx_batch_opt
     const bool keep_engine = opts && opts->keep_engine;
     const EngineKey key = engine_key(*args, eo);
     const uint64_t N = args->size;
-    std::unique_ptr<Engine> eng;
-    // declared after the engine, so destroyed first on every exit path: no
-    // prologue work may still be queued on its stream when the engine frees
-    // the buffers it uses (a DM without trials is never waited for)
+    // destroyed after the engine, whose batches read the series
     std::unique_ptr<CallBuffers> buf;
+    std::unique_ptr<Engine> eng;
+    // destroyed first on every exit path: no prologue work may still be queued
+    // on its stream when the engine frees the buffers it uses (a DM without
+    // trials is never waited for)
+    struct DrainGuard {
+      std::unique_ptr<CallBuffers>& b;
+      ~DrainGuard() {
+        if (b && b->ps) (void)hipStreamSynchronize(b->ps);
+      }
+    } drain{buf};
     if (!keep_engine || !take_kept(key, eng, buf, s)) {
       drop_kept_series();
       hip_check(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), "batch stream");
@@ -476,8 +483,8 @@ extern "C" int psx_batch_search(const psx_search_args* args, const psx_batch_opt
       keep(std::move(eng), std::move(buf), s, key);
       s = nullptr;
     } else {
-      buf.reset();
       eng.reset();
+      buf.reset();
     }
     release();
     return psx::search::flatten(flat, out, cap, count) == PSX_OK ? psx::ok() : PSX_ERR_OVERFLOW;
