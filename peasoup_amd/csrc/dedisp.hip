@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "dedisp_pitch.hpp"
 #include "trace.hpp"
 #include "psx.h"
 
@@ -154,7 +155,7 @@ __global__ void __launch_bounds__(kB) k_unpack_t(const uint8_t* __restrict__ in,
 // spill them into 32-bit sums every kFlush channels.  All sums are exact
 // integers.
 constexpr int kDms = 4;             // DM trials per wave
-constexpr int kTileSamps = 1024;    // samples per wave: four dwords per lane
+using psx::kTileSamps;              // samples per wave: four dwords per lane
 
 template <int NBITS, bool WIDE>
 struct DmSums {
@@ -519,19 +520,6 @@ int launch_lds(const SumArgs& a, hipStream_t s) {
   PSX_CHECK_LAUNCH("k_dedisp_lds");
   return PSX_OK;
 }
-// Dwords per shifted copy for groups of `per` DM trials of an ascending list
-// (0: does not ascend): delays of one channel differ inside a group by at most
-// the DM difference times the largest table entry, plus the two roundings.
-uint32_t staged_pitch(const float* dm, uint32_t ndm, uint32_t per, float tmax) {
-  double spread = 0;
-  for (uint32_t d = 1; d < ndm; ++d)
-    if (!(dm[d] >= dm[d - 1])) return 0;
-  for (uint32_t g = 0; g < ndm; g += per)
-    spread = std::max(spread, ((double)dm[std::min(g + per, ndm) - 1] - (double)dm[g]) * (double)tmax * (1 + 1e-6) + 2);
-  // the tile, the spread, one dword past them for the shifts, whole 16-byte steps
-  const double dwords = std::ceil((kTileSamps + spread) / 4) + 1;
-  return dwords > 1e6 ? UINT32_MAX : ((uint32_t)dwords + 3) / 4 * 4;
-}
 template <int NBITS>
 int launch_sum(SumArgs a, const float* dm_list, float tmax, hipStream_t s) {
   constexpr uint32_t kMax = (1u << NBITS) - 1u;
@@ -545,10 +533,10 @@ int launch_sum(SumArgs a, const float* dm_list, float tmax, hipStream_t s) {
   // stretch's bytes in registers and lose to the direct form (40 DMs of 512
   // 4-bit channels to DM 250: 1.63 ms against 0.41)
   uint32_t nw = a.ndm > 16 && (a.ndm + 31) / 32 * tiles >= 512 ? 8 : 4;
-  a.pitch = staged_pitch(dm_list, a.ndm, kDms * nw, tmax);
+  a.pitch = psx::staged_pitch(dm_list, a.ndm, kDms * nw, tmax);
   if (nw == 8 && a.pitch > kMaxPitch) {
     nw = 4;
-    a.pitch = staged_pitch(dm_list, a.ndm, kDms * nw, tmax);
+    a.pitch = psx::staged_pitch(dm_list, a.ndm, kDms * nw, tmax);
   }
   if (a.nrows > 0 && a.ndm > 2 && a.pitch && a.pitch <= kMaxPitch) {
     if constexpr (kCanWide)
