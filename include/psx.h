@@ -284,8 +284,10 @@ typedef struct psx_batch_opts {
 /* Spectrum hand-over of the batched path.  AUTO: a multi-pass plan whose
  * last pass has a contiguous-row kernel writes contiguous rows and the
  * spectrum pass reads that transposed layout; NATURAL: always natural bin
- * order; ROWS: the transposed layout, an error when the plan has none.  All
- * three give identical spectra for the same FFT decomposition. */
+ * order; ROWS: the transposed layout, an error when the plan has none (without
+ * a decomposition of the caller's: the default one, else the two passes with
+ * the longest last one).  All three give identical spectra for the same FFT
+ * decomposition. */
 enum { PSX_SPECTRUM_AUTO = 0, PSX_SPECTRUM_NATURAL = 1, PSX_SPECTRUM_ROWS = 2 };
 
 /* Harmonic-sum pass of the batched path (harmonic_sum_kernel + PeakFinder,

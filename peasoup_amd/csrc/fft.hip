@@ -513,6 +513,30 @@ static void two_pass_tiles(Decomp& d, uint32_t batch) {
   if (k1 && k1->lds <= 160 * 1024) d.C[1] = c1;
 }
 
+// The two-pass split with the longest last pass (M1 = 0: none).
+static void longest_last(uint64_t M, uint64_t& M1, uint64_t& M2) {
+  M1 = M2 = 0;
+  for (uint64_t m = 32; m <= 4096 && m < M; m = (m % 3 == 0) ? (m / 3) * 4 : m + m / 2) {
+    if (M % m || !len_supported(m, true) || !len_supported(M / m, true)) continue;
+    if (m > M1) {
+      M1 = m;
+      M2 = M / m;
+    }
+  }
+}
+
+bool rows_decomp(uint64_t M, Decomp& d) {
+  d = Decomp();
+  uint64_t M1, M2;
+  if (!valid_complex_len(M) || len_supported(M, false)) return false;
+  longest_last(M, M1, M2);
+  if (!M1 || M2 > 2048) return false;
+  d.npass = 2;
+  d.L[0] = (int)M2;
+  d.L[1] = (int)M1;
+  return pick_tiles(d) && find_kernel(d.L[1], d.C[1], PM_CONTIG, false);
+}
+
 // Default decomposition: one pass when a single-workgroup kernel exists, else
 // two passes of about equal length, the strided one the largest power of two
 // that is at most 1,024 and no longer than the contiguous last one (whose
@@ -553,15 +577,7 @@ bool default_decomp(uint64_t M, Decomp& d, uint32_t batch) {
     return pick_tiles(d);
   }
   uint64_t bM1 = 0, bM2 = 0;
-  for (uint64_t M1 = 32; M1 <= 4096 && M1 < M; M1 = (M1 % 3 == 0) ? (M1 / 3) * 4 : M1 + M1 / 2) {
-    if (M % M1) continue;
-    const uint64_t M2 = M / M1;
-    if (!len_supported(M1, true) || !len_supported(M2, true)) continue;
-    if (M1 > bM1) {
-      bM1 = M1;
-      bM2 = M2;
-    }
-  }
+  longest_last(M, bM1, bM2);
   auto two = [&]() {
     d.npass = 2;
     d.L[0] = (int)bM2;

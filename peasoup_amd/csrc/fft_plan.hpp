@@ -23,6 +23,11 @@ struct Decomp {
 bool valid_complex_len(uint64_t m);
 // batch: transforms per launch (sets the column tiles, not the lengths).
 bool default_decomp(uint64_t M, Decomp& d, uint32_t batch);
+// A two-pass decomposition whose last pass has a row-layout kernel, for callers
+// that ask for that layout where the default one has none (false: no such
+// split).  The default's even splits end on passes of 128 to 768 points, most
+// of them without one; this is the split with the longest last pass.
+bool rows_decomp(uint64_t M, Decomp& d);
 bool pick_tiles(Decomp& d);
 bool decomp_supported(const Decomp& d);
 // Roots W_n^k of the real length n as a two-level table: W = hi[k>>shift]*lo[k&mask].

@@ -74,11 +74,21 @@ Engine::Engine(const psx_search_args& a, const EngineOptions& opt, hipStream_t s
   if (cap < kPrefix) cap = kPrefix;
   pstride = round_up((int64_t)nb, 64);
   psx_ok(psx::fft::plan_create_with(N, PSX_FFT_R2C, B, opt.decomp, &plan), "batched R2C plan");
-  rt = psx::fft::root_table(plan);
   if (opt.spectrum_layout < PSX_SPECTRUM_AUTO || opt.spectrum_layout > PSX_SPECTRUM_ROWS)
     throw std::runtime_error("spectrum_layout must be PSX_SPECTRUM_AUTO, _NATURAL or _ROWS");
-  const bool rows_ok =
-      psx::fft::rows_layout(plan, &rows_R, &rows_L) && rows_L % 64 == 0 && rows_R % 2 == 0 && rows_R >= 4;
+  auto has_rows = [&] {
+    return psx::fft::rows_layout(plan, &rows_R, &rows_L) && rows_L % 64 == 0 && rows_R % 2 == 0 && rows_R >= 4;
+  };
+  bool rows_ok = has_rows();
+  // ROWS without a plan of the caller's: a plan that has them
+  psx::fft::Decomp rows_plan;
+  if (opt.spectrum_layout == PSX_SPECTRUM_ROWS && !rows_ok && !opt.decomp && psx::fft::rows_decomp(M, rows_plan)) {
+    psx_fft_plan_destroy(plan);
+    plan = nullptr;
+    psx_ok(psx::fft::plan_create_with(N, PSX_FFT_R2C, B, &rows_plan, &plan), "batched R2C plan");
+    rows_ok = has_rows();
+  }
+  rt = psx::fft::root_table(plan);
   if (opt.spectrum_layout == PSX_SPECTRUM_ROWS && !rows_ok)
     throw std::runtime_error("spectrum_layout ROWS: this FFT plan has no row-layout last pass");
   rows_out = rows_ok && opt.spectrum_layout != PSX_SPECTRUM_NATURAL;
