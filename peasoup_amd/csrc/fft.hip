@@ -540,12 +540,11 @@ bool rows_decomp(uint64_t M, Decomp& d) {
 // Default decomposition: one pass when a single-workgroup kernel exists, else
 // two passes of about equal length, the strided one the largest power of two
 // that is at most 1,024 and no longer than the contiguous last one (whose
-// rows are read and written whole), but 512 for 256, and 2,048 before 1,536
-// for 1,024 before 3,072.  Against the longest last pass, which
+// rows are read and written whole), but 512 for 256.  Against the longest last pass, which
 // this rule replaces below 2^23 samples (R2C of one transform and, in the
 // batched search, us per trial): 2^17 17.2 and 1.68 -> 12.7 and 0.95, 2^20
 // 21.2 and 5.10 -> 17.4 and 5.01, 2^21 31.1 and 10.93 -> 26.3 and 9.80, 3*2^17
-// 27.1 and 4.28 -> 15.4 and 2.05, 3*2^21 65.3 and 36.1 -> 44.9 and 27.6.
+// 27.1 and 4.28 -> 15.4 and 2.05, 3*2^21 65.3 and 36.1 -> 43.9 and 27.9.
 // Longer: the split with the longest last pass while the strided pass is at
 // most 2,048 points (2^24: 2,048 x 4,096), else three passes as below.
 bool default_decomp(uint64_t M, Decomp& d, uint32_t batch) {
@@ -568,9 +567,7 @@ bool default_decomp(uint64_t M, Decomp& d, uint32_t batch) {
     // 19.8, 82 us, 3*2^16 15.5, 22.8, 74 -> 14.3, 20.1, 64, 3*2^17 17.0, 28.8,
     // 133 -> 15.4, 26.3, 131; searches in batches of 8 and 64 4% less).  At
     // 2^17 batches of 8 lose more (6.2 -> 6.9 us per trial) than R2C gains.
-    // Rows of 3,072 points leave one workgroup per CU; behind 2,048 points they
-    // halve (searches of 3*2^21 samples 17.8 -> 17.4 ms, one R2C 43.9 -> 44.9 us).
-    const bool longer = (M2 == 256 && M1 > 256) || M1 == 3072;
+    const bool longer = M2 == 256 && M1 > 256;
     d.L[0] = (int)(longer ? 2 * M2 : M2);
     d.L[1] = (int)(longer ? M1 / 2 : M1);
     two_pass_tiles(d, batch);

@@ -1,13 +1,12 @@
 """Default FFT plans around the lengths whose strided pass of 256 points gives
-way to one of 512 before shorter rows, and at the one whose rows of 3,072 points
-do to 1,536."""
+way to one of 512 before shorter rows."""
 import numpy as np
 import pytest
 
 import peasoup_amd as P
 
 SIZES = [(1 << 17, "256/C8x256"), (1 << 18, "512/C8x256"), (3 << 16, "512/C8x192"), (3 << 17, "512/C8x384"),
-         (1 << 19, "512/C8x512"), (3 << 21, "2048/C8x1536")]
+         (1 << 19, "512/C8x512")]
 
 
 @pytest.mark.parametrize("n", [n for n, _ in SIZES])
