@@ -314,8 +314,10 @@ int psx_batch_search(const psx_search_args* args, const psx_batch_opts* opts, co
 /* Frees the engine a psx_batch_search call with keep_engine left behind
  * (its device buffers, FFT plans and launch graphs, and the call's dereddened
  * series where they take no more device memory than the engine; a call that
- * builds another engine frees those series first; one engine is kept per
- * process, replaced by the next keeping call with other arguments).  No
+ * builds another engine frees those series first, and so does an allocation of
+ * this library that finds no device memory, before it is tried again; one
+ * engine is kept per process, replaced by the next keeping call with other
+ * arguments).  No
  * counterpart in the reference, whose Worker builds its transforms per DM
  * (pipeline_multi.cu:111-145); for pipelines that search many segments of
  * one shape. */

@@ -19,6 +19,14 @@ int fail(int code, const char* fmt, ...);
 // Clears the thread-local error message and returns PSX_OK.
 int ok();
 
+// hipMalloc for every device buffer of the library.  The batched search keeps
+// its series between calls; an allocation that finds no memory has them freed
+// and is tried again, so that whatever fitted beside the engine alone still
+// does.
+hipError_t device_malloc(void** ptr, uint64_t bytes);
+// Frees the kept series; false: none were kept.
+bool drop_kept_series();
+
 inline hipStream_t as_stream(psx_stream s) { return reinterpret_cast<hipStream_t>(s); }
 
 // Grid size for a grid-stride loop over n items with `per_block` items per

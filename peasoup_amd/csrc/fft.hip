@@ -758,7 +758,7 @@ int build_passes(psx_fft_plan* p, bool device_tables) {
   size_t rlo = 0, rhi = 0;
   append_two(p->n, rsh, rlo, rhi);
   if (device_tables) {
-    PSX_CHECK_HIP(hipMalloc(&p->tables, size * sizeof(float2)));
+    PSX_CHECK_HIP(psx::device_malloc((void**)&p->tables, size * sizeof(float2)));
     k_roots<<<dim3(64, runs.n), 256>>>(p->tables, runs);
     PSX_CHECK_LAUNCH("k_roots");
     // plans run on any stream
@@ -902,7 +902,7 @@ int plan_create_with(uint64_t n, int kind, uint32_t batch, const Decomp* forced,
   if (!rc) {
     const bool need_work = own_work && ((kind == PSX_FFT_C2R) || p->d.npass > 1);
     if (need_work) {
-      hipError_t e = hipMalloc(&p->work, sizeof(float2) * p->M * batch);
+      hipError_t e = psx::device_malloc((void**)&p->work, sizeof(float2) * p->M * batch);
       if (e != hipSuccess) rc = psx::fail(PSX_ERR_ALLOC, "FFT work buffer: %s", hipGetErrorString(e));
     }
   }

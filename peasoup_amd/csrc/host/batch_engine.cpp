@@ -26,7 +26,7 @@ void psx_ok(int rc, const char* what) {
 }
 template <class T>
 void dalloc(T** p, uint64_t n) {
-  hip_ok(hipMalloc((void**)p, sizeof(T) * (n ? n : 1)), "hipMalloc");
+  hip_ok(psx::device_malloc((void**)p, sizeof(T) * (n ? n : 1)), "hipMalloc");
 }
 template <class T>
 void halloc(T** p, uint64_t n) {

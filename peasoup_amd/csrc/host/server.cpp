@@ -365,10 +365,10 @@ bool psx_server::admit_one(Request* r) {
     es->spare = nullptr;
     es->spare_bytes = 0;
   } else {
-    hipError_t e = hipMalloc(&r->d_tims, r->bytes);
+    hipError_t e = psx::device_malloc((void**)&r->d_tims, r->bytes);
     if (e != hipSuccess && spare) {
       drop_spares();
-      e = hipMalloc(&r->d_tims, r->bytes);
+      e = psx::device_malloc((void**)&r->d_tims, r->bytes);
     }
     if (e != hipSuccess) {
       (void)hipGetLastError();

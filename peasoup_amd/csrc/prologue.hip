@@ -319,10 +319,10 @@ int work_create(uint64_t n, uint32_t G, Work& w) {
   w.c25 = w.c5 / 5;
   w.c125 = w.c25 / 5;
   w.med_stride = w.c5 + w.c25 + w.c125;
-  PSX_CHECK_HIP(hipMalloc(&w.med, std::max<uint64_t>(1, G * w.med_stride) * sizeof(float)));
-  PSX_CHECK_HIP(hipMalloc(&w.partial, (uint64_t)G * kPartials * sizeof(double2)));
-  PSX_CHECK_HIP(hipMalloc(&w.res, G * sizeof(Result)));
-  PSX_CHECK_HIP(hipMalloc(&w.zmask, (nb / 32 + 1) * sizeof(uint32_t)));
+  PSX_CHECK_HIP(psx::device_malloc((void**)&w.med, std::max<uint64_t>(1, G * w.med_stride) * sizeof(float)));
+  PSX_CHECK_HIP(psx::device_malloc((void**)&w.partial, (uint64_t)G * kPartials * sizeof(double2)));
+  PSX_CHECK_HIP(psx::device_malloc((void**)&w.res, G * sizeof(Result)));
+  PSX_CHECK_HIP(psx::device_malloc((void**)&w.zmask, (nb / 32 + 1) * sizeof(uint32_t)));
   return PSX_OK;
 }
 

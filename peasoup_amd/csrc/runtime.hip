@@ -24,6 +24,16 @@ int ok() {
   return PSX_OK;
 }
 
+hipError_t device_malloc(void** ptr, uint64_t bytes) {
+  hipError_t e = hipMalloc(ptr, bytes);
+  if (e == hipErrorOutOfMemory && drop_kept_series()) {
+    (void)hipGetLastError();
+    e = hipMalloc(ptr, bytes);
+  }
+  if (e != hipSuccess) (void)hipGetLastError();  // reported by the return value
+  return e;
+}
+
 }  // namespace psx
 
 using psx::as_stream;
@@ -70,10 +80,9 @@ extern "C" int psx_malloc(void** ptr, uint64_t bytes) {
   PSX_REQUIRE(ptr, "psx_malloc: null ptr");
   *ptr = nullptr;
   if (bytes == 0) return psx::ok();
-  hipError_t e = hipMalloc(ptr, bytes);
+  hipError_t e = psx::device_malloc(ptr, bytes);
   if (e != hipSuccess) {
     *ptr = nullptr;
-    (void)hipGetLastError();
     return psx::fail(PSX_ERR_ALLOC, "hipMalloc(%llu) failed: %s", (unsigned long long)bytes, hipGetErrorString(e));
   }
   return psx::ok();
