@@ -401,8 +401,8 @@ typedef struct psx_request_status {
 } psx_request_status;
 
 typedef struct psx_server_stats {
-  uint64_t used_bytes, budget_bytes; /* used: engines and admitted requests; the series buffer of each
-                                        engine's last request, kept for its next, comes on top, within
+  uint64_t used_bytes, budget_bytes; /* used: engines and admitted requests; one finished request's series
+                                        buffer per engine, kept for its next ones, comes on top, within
                                         the budget */
   uint32_t waiting, active, engines;
   uint64_t completed, failed, trials_done;

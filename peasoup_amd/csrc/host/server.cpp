@@ -94,17 +94,20 @@ struct PinnedResults {
   PinnedResults& operator=(const PinnedResults&) = delete;
 };
 
+constexpr uint32_t kSpareIdle = 8;
+
 struct EngineState {
   PinnedResults res;  // declared first: outlives the engine, whose destructor drains the stream
   std::unique_ptr<Engine> eng;
   hipStream_t stream = nullptr;
   hipEvent_t mark = nullptr;  // the engine stream's work so far (mixed dispatch waits on it)
   uint64_t bytes = 0;
-  // the series buffer of the engine's last finished request, for its next one
-  // of that size: hipFree waits for the device (0.25 ms on average, up to
-  // 5 ms, while the other engines' next batches waited to be launched)
+  // a finished request's series buffer, for the next request of that size:
+  // hipFree waits for the device (0.25 ms on average, up to 5 ms, while the
+  // other engines' next batches waited to be launched)
   float* spare = nullptr;
   uint64_t spare_bytes = 0;
+  uint32_t spare_idle = 0;           // smaller requests ended since the buffer was kept
   std::deque<TrialRef> queue;        // trials waiting for a batch
   std::deque<std::vector<TrialRef>> inflight;  // trials of each submitted batch
   clk::time_point last_used;
@@ -455,13 +458,19 @@ void psx_server::finish(Request* r) {
   psx::search::flatten(flat, r->result.data(), (uint32_t)r->result.size(), &cnt);
   r->per_trial.clear();
   r->zap.reset();
-  // every trial that read the series has been collected; the larger of two
-  // buffers stays with the engine
+  // every trial that read the series has been collected.  The larger of two
+  // buffers stays with the engine, so that requests of two sizes in turn still
+  // have one of them back (two beams of 32 and 16 DMs served together: 3.5 ms a
+  // round, 3.8 where the last one's buffer stays), but not for ever: once
+  // kSpareIdle smaller requests have ended without it being taken, their own
+  // takes its place
   EngineState* es = r->es;
-  if (es->spare_bytes < r->bytes) {
+  if (r->bytes > es->spare_bytes || (r->bytes < es->spare_bytes && ++es->spare_idle >= kSpareIdle)) {
     std::swap(es->spare, r->d_tims);
-    spare += r->bytes - es->spare_bytes;
+    spare -= es->spare_bytes;
+    spare += r->bytes;
     es->spare_bytes = r->bytes;
+    es->spare_idle = 0;
   }
   (void)hipFree(r->d_tims);
   r->d_tims = nullptr;
