@@ -64,15 +64,18 @@ def test_stretches_fit(pitches, log_delay):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("delay", [1017, 5000, (1 << 24) + 3, (1 << 28) + 77])
-def test_long_delays(psx, delay):
+@pytest.mark.parametrize("delay,spread", [
+    (1017, 1016), (1017, 1000),  # the widest spread staged (512 dwords)
+    (5000, 1000), ((1 << 24) + 3, 1000), ((1 << 28) + 77, 960),
+])
+def test_long_delays(psx, delay, spread):
     """Two channels, the second delayed by up to `delay` samples."""
     import peasoup_amd.sigproc as sigproc
     dt, f0, df = f32(0.000256), f32(1500.0), f32(-150.0)
     tab = sigproc.delay_table(2, dt, f0, df)
     ndm = 16
     top = delay / float(tab[1])
-    dms = np.linspace(max(0.0, top - 1000 / float(tab[1])), top, ndm).astype(f32)
+    dms = np.linspace(max(0.0, top - spread / float(tab[1])), top, ndm).astype(f32)
     lag = np.rint(dms * tab[1]).astype(np.int64)
     nout = 2500
     n = int(lag[-1]) + nout
