@@ -195,10 +195,8 @@ class Zapper {
   void zap(DeviceFourierSeries<psx_c32>& fseries) {
     zap(fseries.get_data(), fseries.get_bin_width(), fseries.get_nbins());
   }
-  void zap(psx_c32* fseries, float bin_width, unsigned int nbins) {
-    peasoup::check(psx_zap_birdies(fseries, d_birdies, d_widths, (uint32_t)birdies.size(), bin_width, nbins, stream),
-                   "Zapper::zap");
-  }
+  void zap(psx_c32* fseries, float bin_width, unsigned int nbins) { zap_on(fseries, bin_width, nbins, stream); }
+  // zap on a stream of the caller's
   void zap_on(psx_c32* fseries, float bin_width, uint64_t nbins, psx_stream s) const {
     peasoup::check(psx_zap_birdies(fseries, d_birdies, d_widths, (uint32_t)birdies.size(), bin_width, nbins, s),
                    "Zapper::zap");
