@@ -1049,7 +1049,8 @@ int launch_spec_rows(const float2* Y, float* P, uint32_t R, uint32_t L, int64_t 
                      const TrialDesc* d_descs, uint32_t ntr, hipStream_t s, const SpecBound* bound) {
   if (R < 4 || R % 2 || L % kColTile || (uint64_t)R * L > 0x7FFFFFFFull || pstride < (int64_t)R * L + 1)
     return psx::fail(PSX_ERR_ARG, "spec_rows: unsupported layout %u x %u", R, L);
-  // the bound pairs of a tile's rows need an even tile base row minus one
+  // a tile's bounds lie around its even rows, and so does row R/2's (R - r is
+  // even with r; R/2 is the edge workgroups')
   if (bound && (R % 4 || bound->qstride < bound_stride(pstride)))
     return psx::fail(PSX_ERR_ARG, "spec_rows: unsupported bound layout %u x %u", R, L);
   // row tiles of rows [1, R/2), then one row of workgroups for the edge bins

@@ -95,8 +95,9 @@ Engine::Engine(const psx_search_args& a, const EngineOptions& opt, hipStream_t s
   if (opt.harmonic_pass != PSX_HARMONIC_BOUND && opt.harmonic_pass != PSX_HARMONIC_EXACT)
     throw std::runtime_error("harmonic_pass must be PSX_HARMONIC_BOUND or PSX_HARMONIC_EXACT");
   bound = opt.harmonic_pass == PSX_HARMONIC_BOUND && F > 0;
-  // the row-layout pass pairs bins (2u, 2u+1) by rows, which needs R % 4 == 0
-  // (true of every plan with that layout: R is 2^k or 3*2^k, k >= 5)
+  // the row-layout pass bounds the bins (2u-1, 2u, 2u+1) from three neighbouring
+  // rows around an even one, lower and upper alike, which needs R/2 even (true
+  // of every plan with that layout: R is 2^k or 3*2^k, k >= 5)
   fused = bound && rows_out && rows_R % 4 == 0;
   dalloc(&Z, M * B);
   if (!fused) dalloc(&P, (uint64_t)pstride * B + kHarmWaveBins);

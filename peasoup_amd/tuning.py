@@ -4,7 +4,9 @@ For a series length n the tuner times candidate schedules - FFT
 decompositions (pass lengths and column tiles) and trials per batch - with
 psx_batch_profile (HIP events around every fused launch) and keeps the
 fastest per trial.  Results are stored per (device name, n) in
-peasoup_amd/tuned.json (shipped, measured on MI355X) and in the user cache
+peasoup_amd/tuned.json (shipped, measured on MI355X with ROCm's own HIP runtime,
+whose device name is empty: "gfx950-256CU"; under the runtime that torch loads
+device_info names the card otherwise and finds no entry) and in the user cache
 (~/.cache/peasoup_amd/tuned.json) for new shapes.  Measured HBM traffic of
 profiled kernels (rocprofv3 FETCH_SIZE/WRITE_SIZE) is kept in
 profiles/traffic.json and reported by bench.py.
